@@ -62,6 +62,12 @@ int gemv16_dispatch(const uint16_t* A, const GemvShard* shards, int nshards, int
 size_t gemm_grouped_shard_bytes(int rows, int ic, int oc);
 int gemm_grouped_dispatch(const uint16_t* A, const GemvShard* shards, int nshards, int rows, char* ws,
                           size_t ws_bytes, hipStream_t stream, const char* what = "exl3_gemm_grouped");
+// exl3_gemm and exl3_gemm_grouped up to this many rows run the K-split decode-GEMM (gemm_ks.hip;
+// gemm.hip has both sides' times).
+constexpr int KS_MAX_ROWS = 512;
+size_t gemm_ks_shard_bytes(int rows, int ic, int oc);
+int gemm_ks_dispatch(const uint16_t* A, const GemvShard* shards, int nshards, int rows, char* ws, size_t ws_bytes,
+                     hipStream_t stream, const char* what);
 int gemm_sk_cus();
 // The launch's tile counters, the first sk_ntiles(rows, oc) words of ws, must be 0 when it
 // starts (exl3_gemm's Hadamard pass clears them).

@@ -702,6 +702,7 @@ size_t gemm_sk_slot_bytes(int rows, int oc) { return sk_single_bytes(rows, oc, g
 
 size_t gemm_grouped_shard_bytes(int rows, int ic, int oc)
 {
+    if (rows <= KS_MAX_ROWS) return gemm_ks_shard_bytes(rows, ic, oc);
     return sk_grouped_bytes_bm(gemm_sk_bm(rows), rows, ic, oc, gemm_sk_cus());
 }
 
@@ -805,6 +806,7 @@ static int sk_grouped_dispatch(const uint16_t* A, const GemvShard* shards, int n
 int gemm_grouped_dispatch(const uint16_t* A, const GemvShard* shards, int nshards, int rows, char* ws,
                           size_t ws_bytes, hipStream_t stream, const char* what)
 {
+    if (rows <= KS_MAX_ROWS) return gemm_ks_dispatch(A, shards, nshards, rows, ws, ws_bytes, stream, what);
     switch (gemm_sk_bm(rows)) {
     case 32: return sk_grouped_dispatch<32>(A, shards, nshards, rows, ws, ws_bytes, what, stream);
     case 48: return sk_grouped_dispatch<48>(A, shards, nshards, rows, ws, ws_bytes, what, stream);

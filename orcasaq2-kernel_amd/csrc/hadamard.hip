@@ -16,44 +16,6 @@ namespace exl3 {
 
 constexpr int HAD_WAVES = 4;
 
-// v from lane l ^ 4 within each 16-lane row: banks 0 and 2 (lane bit 2 clear) read lane l + 4
-// (row_shl:4), banks 1 and 3 read lane l - 4 (row_shr:4).
-__device__ __forceinline__ float had_xor4(float v)
-{
-    const int x = __builtin_bit_cast(int, v);
-    int t = __builtin_amdgcn_update_dpp(0, x, 0x104, 0xf, 0x5, false);
-    t = __builtin_amdgcn_update_dpp(t, x, 0x114, 0xf, 0xa, false);
-    return __builtin_bit_cast(float, t);
-}
-
-template <int D>
-__device__ __forceinline__ float had_xor(float v)
-{
-    const int x = __builtin_bit_cast(int, v);
-    if constexpr (D == 1) return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(x, 0xB1, 0xf, 0xf, false));   // quad_perm [1,0,3,2]
-    else if constexpr (D == 2) return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(x, 0x4E, 0xf, 0xf, false));  // quad_perm [2,3,0,1]
-    else if constexpr (D == 4) return had_xor4(v);
-    else return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(x, 0x128, 0xf, 0xf, false));  // row_ror:8
-}
-
-__device__ __forceinline__ void had_unpack(const uint4& q, float (&v)[8])
-{
-    const uint32_t w[4] = {q.x, q.y, q.z, q.w};
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        v[2 * i] = (float)__builtin_bit_cast(_Float16, (uint16_t)(w[i] & 0xffffu));
-        v[2 * i + 1] = (float)__builtin_bit_cast(_Float16, (uint16_t)(w[i] >> 16));
-    }
-}
-
-template <int D>
-__device__ __forceinline__ void had_lane_stage(float (&v)[8], int lane)
-{
-    const float sg = (lane & D) ? -1.f : 1.f;
-#pragma unroll
-    for (int i = 0; i < 8; i++) v[i] = __builtin_fmaf(v[i], sg, had_xor<D>(v[i]));
-}
-
 // Words zero[0 .. nzero) to 0 by workgroup 0 (before any of its lanes leaves).
 __device__ __forceinline__ void had_zero(uint32_t* zero, int nzero)
 {
@@ -78,19 +40,7 @@ __global__ __launch_bounds__(64 * HAD_WAVES) void had_r_128_kernel(
 #pragma unroll
         for (int i = 0; i < 8; i++) v[i] *= p[i];
     }
-#pragma unroll
-    for (int d = 1; d < 8; d <<= 1)
-#pragma unroll
-        for (int i = 0; i < 8; i++)
-            if (!(i & d)) {
-                const float a = v[i], b = v[i + d];
-                v[i] = a + b;
-                v[i + d] = a - b;
-            }
-    had_lane_stage<1>(v, lane);
-    had_lane_stage<2>(v, lane);
-    had_lane_stage<4>(v, lane);
-    had_lane_stage<8>(v, lane);
+    had16_stages(v, lane);
     float f[8];
 #pragma unroll
     for (int i = 0; i < 8; i++) f[i] = 0.08838834764831845f * scale;   // 1/sqrt(128)

@@ -23,6 +23,7 @@
 #include <string>
 #include <vector>
 
+#include "../gemm_ks_plan.h"
 #include "../gemm_sk_plan.h"
 #include "../gemv16_plan.h"
 #include "../gemv1_plan.h"
@@ -1149,9 +1150,274 @@ void g16_replay_finish(G16World& W, const GemvShard* shards, const G1Group& a, c
     }
 }
 
+// ================================================================ K-split decode-GEMM
+
+struct KsWorld {
+    int rows, ic, cols;
+    std::vector<ShardSpec> sh;
+    std::vector<int> col0;
+    size_t ws_bytes;
+    std::vector<uint8_t> out;
+    std::vector<std::pair<long, long>> regions;   // [begin, end) of each workspace use
+    long loads = 0, pieces = 0, slot_writes = 0;
+};
+
+void ks_region(KsWorld& W, const void* p, long bytes, const char* what)
+{
+    need_in(p, bytes, B_WS, (long)W.ws_bytes, what);
+    const long b = off_of(p), e = b + bytes;
+    for (auto& r : W.regions)
+        if (b < r.second && r.first < e) fail("%s: workspace bytes [%ld, %ld) overlap [%ld, %ld)", what, b, e, r.first, r.second);
+    W.regions.push_back({b, e});
+}
+
+// Row r0 .. r0 + n - 1 of column group cg of shard si of a launch stored.
+void ks_store_rows(KsWorld& W, const GemvShard* shards, const KsArgs& a, int si, int cg, int r0, int n)
+{
+    const KsShard& S = a.sh[si];
+    int i = 0;
+    while (shards[i].trellis != S.trellis) i++;
+    need_in(S.svh + cg * 128, 256, B_SVH + i, 2l * shards[i].oc, "ks svh");
+    for (int r = r0; r < r0 + n; r++) {
+        if (r >= a.rows) continue;
+        need_in(S.C + (long)r * S.ldc + cg * 128, 256, B_C, 2l * W.rows * W.cols, "ks output");
+        for (int c = 0; c < 128; c++) {
+            const long o = off_of(S.C + (long)r * S.ldc + cg * 128 + c) / 2;
+            if (W.out[o]++) fail("ks output row %d shard %d column %d written twice", r, i, cg * 128 + c);
+        }
+    }
+}
+
+void ks_check_lds(int mt)
+{
+    const int NP = KS_NP, floats = ks_lds(mt) / 4;
+    std::vector<char> seen(floats, 0);
+    for (int w = 0; w < 2 * NP; w++)
+        for (int lane = 0; lane < 64; lane++)
+            for (int h = 0; h < 2; h++)
+                for (int j = 0; j < 4; j++) {
+                    const int i = ks_red(w >> 1, 64 * (w & 1) + 32 * h + (lane & 31), 2 * j + (lane >> 5));
+                    if (i < 0 || i % 4 || i + 4 > floats) fail("ks staging store at float %d of %d", i, floats);
+                    if (seen[i]++) fail("ks staging float %d stored twice", i);
+                }
+    for (int w = 0; w < NP; w++)
+        for (int idx = 0; idx < 1024; idx++)
+            if (seen[ks_red(w, idx & 127, idx >> 7)] != 1) fail("ks staging read of an unwritten quad");
+    std::vector<char> col(128, 0);
+    for (int c = 0; c < 128; c++) {
+        const int o = ks_out_col(c);
+        if (o < 0 || o > 127 || col[o]++) fail("ks output column of position %d is %d", c, o);
+    }
+    if (32 * KS_LDC > floats) fail("ks output staging beyond LDS");
+    // the ring: every stage's loads land once, inside LDS, where the reads look for them
+    for (int K = 1; K <= 8; K++) {
+        std::vector<char> hit(ks_lds(mt) / 4, 0);
+        for (int st = 0; st < ks_nb(mt); st++)
+            for (int w = 0; w < 2 * NP; w++) {
+                for (int t = 0; t < mt; t++)
+                    for (int lane = 0; lane < 64; lane++)
+                        for (int e = 0; e < 4; e++)
+                            if (hit.at((ks_stage_a(mt, st, w >> 1) + (w & 1) * mt * 1024 + t * 1024 + 16 * lane) / 4 + e)++)
+                                fail("ks A stage word loaded twice");
+                // word loads: each run's lanes side by side, inside the wave's area
+                for (int r = 0; r < ks_w_runs(K); r++)
+                    for (int lane = 0; lane < 64; lane++)
+                        for (int e = 0; e < (K == 1 ? 1 : 4); e++) {
+                            const int o = 1024 * r + (K == 1 ? 4 : 16) * lane + 4 * e;
+                            if (o + 4 > KS_WBYTES || hit.at((ks_stage_w(mt, st, w) + o) / 4)++) fail("ks word stage overlaps");
+                        }
+                for (int lane = 0; lane < 64; lane++)
+                    for (int i = 0; i < K; i++) {
+                        // word i of the chunk is at run r's place of the words it loads
+                        const int r = i >= 4, e = i - ks_w_run(K, r, lane);
+                        if (e < 0 || e >= (K == 1 ? 1 : 4) || ks_w_off(K, i, lane) != 1024 * r + (K == 1 ? 4 : 16) * lane + 4 * e)
+                            fail("ks word %d of lane %d (K %d) read elsewhere", i, lane, K);
+                    }
+            }
+    }
+}
+
+void ks_replay(KsWorld& W, const GemvShard* shards, const KsLaunch& L)
+{
+    const KsArgs& a = *L.args;
+    const KsPrepArgs& p = *L.prep;
+    const int mt = L.mt;
+    ks_check_lds(mt);
+    const int NP = KS_NP;
+    int ncg = 0;
+    for (int i = 0; i < a.nshards; i++) ncg += a.sh[i].tc / 8;
+    const int nsegs = a.nrt * ncg;
+    if (L.G < 1 || a.G != L.G || a.full * a.G + a.nrem != nsegs || a.nrem >= a.G || a.mtt != a.nrt * mt || a.mtt * 32 < a.rows)
+        fail("ks launch sizes");
+    // set-up: every fragment chunk written once, by the (row, inputs) its readers expect
+    const long chunks = (long)a.P * a.mtt * 128;
+    std::vector<std::vector<int>> ah(p.nsh, std::vector<int>(chunks, -1));
+    for (int s = 0; s < p.nsh; s++) {
+        if (p.Ah[s] != a.sh[s].Ah) fail("ks set-up writes another buffer than the decode reads");
+        ks_region(W, p.Ah[s], chunks * 16, "ks activations");
+    }
+    if (p.mtt > 65535 || a.nrem > 65535) fail("ks grid");
+    for (int wg = 0; wg < p.nsh * p.nblk * p.mtt; wg++) {
+        const int b = wg % p.nblk, m = wg / p.nblk % p.mtt, s = wg / p.nblk / p.mtt;
+        int i = 0;
+        while (shards[i].suh != p.suh[s]) i++;
+        for (int t = 0; t < 512; t++) {
+            const int row = 4 * (t >> 6) + ((t & 63) >> 4), l16 = t & 15;
+            if (32 * m + row < p.rows) {
+                need_in(p.A + (long)(32 * m + row) * p.ic + b * 128 + 8 * l16, 16, B_X, 2l * W.rows * W.ic, "ks set-up x");
+                need_in(p.suh[s] + b * 128 + 8 * l16, 16, B_SUH + i, 2l * W.ic, "ks set-up suh");
+            }
+            const long c = ks_prep_chunk(p, b, m, row, l16);
+            if (c < 0 || c >= chunks || ah[s][c] >= 0) fail("ks set-up chunk %ld", c);
+            ah[s][c] = (32 * m + row) * (W.ic / 8) + b * 16 + l16;
+        }
+    }
+    for (auto& v : ah)
+        for (int x : v)
+            if (x < 0) fail("ks set-up left a chunk unwritten");
+    const long slot4 = a.nrem ? (long)(a.nrem + a.G) * mt * 1024 : 0;
+    if (slot4) ks_region(W, a.slots, slot4 * 16, "ks slots");
+    std::map<int, std::pair<int, int>> slot_owner;         // s + g -> (split segment, workgroup)
+    std::vector<uint8_t> steps((size_t)nsegs * a.P, 0);
+    std::vector<char> wg_seen(L.G, 0);
+    for (int blk = 0; blk < L.G; blk++) {
+        const int g = ks_logical(blk, L.G);
+        if (g < 0 || g >= L.G || wg_seen[g]++) fail("ks block %d -> workgroup %d", blk, g);
+        for (int round = 0; round < a.full + (a.nrem ? 1 : 0); round++) {
+            const bool split = round == a.full;
+            for (int pair = 0; pair < NP; pair++) {
+                // as the kernel finds them
+                int seg = round * a.G + g, k = pair, nmax = ks_run_max(a.whole);
+                KsCut cut = a.whole;
+                if (split) {
+                    const int j0 = NP * g, s0 = ks_seg_of(a, j0), next = ks_pair0(a, s0 + 1), last0 = std::min(NP, next - j0);
+                    const int s = s0 + (pair >= last0);
+                    k = j0 + pair - (pair >= last0 ? next : ks_pair0(a, s0));
+                    cut = ks_cut(a, s);
+                    nmax = ks_run_max(ks_cut(a, last0 < NP ? s0 + 1 : s0));
+                    seg = a.full * a.G + s;
+                    if (s < 0 || s >= a.nrem || s != ks_seg_of(a, j0 + pair) || k < 0 || k >= ks_npairs(a, s) || last0 < 1 ||
+                        cut.q * ks_npairs(a, s) + cut.r != a.P)
+                        fail("ks workgroup %d pair %d: split segment %d run %d", g, pair, s, k);
+                    if (pair == 0 || pair == last0) {
+                        const long b = ks_slot(s0, g, mt) + (pair ? mt * 1024 : 0);
+                        if (b != ks_slot(s, g, mt) || b < 0 || b + mt * 1024 > slot4) fail("ks slot of segment %d workgroup %d", s, g);
+                        if (!slot_owner.emplace(s + g, std::make_pair(s, g)).second) fail("ks slot %d taken twice", s + g);
+                        W.slot_writes++;
+                    }
+                }
+                const KsSeg sg = ks_seg(a, seg);
+                if (seg >= nsegs || sg.rt >= a.nrt || sg.si >= a.nshards) fail("ks segment %d", seg);
+                const KsShard& S = a.sh[sg.si];
+                if (sg.cg < 0 || sg.cg >= S.tc / 8) fail("ks column group %d of shard %d", sg.cg, sg.si);
+                int i = 0;
+                while (shards[i].trellis != S.trellis) i++;
+                const long words = (long)W.ic / 16 * S.tc * 8 * S.K;
+                const int p0 = ks_run(cut, k), p1 = ks_run(cut, k + 1);
+                if (p1 - p0 > nmax) fail("ks pair of %d steps, %d barriers", p1 - p0, nmax);
+                for (int q = p0; q < p1; q++) {
+                    if (steps[(size_t)seg * a.P + q]++) fail("ks segment %d step %d decoded twice", seg, q);
+                    for (int lane = 0; lane < 64; lane++) {
+                        for (int h = 0; h < 2; h++) {
+                            // the kernel's form: the wave's first step's base, the lane's offset,
+                            // the step stride
+                            const long at = ks_b_word(p0, 0, S.tc, sg.cg, h, S.K) + ks_b_word(0, lane, S.tc, 0, 0, S.K) +
+                                            (long)(q - p0) * 2 * S.tc * 8 * S.K;
+                            need_in(S.trellis + at, 4 * S.K, B_TRELLIS + i, 4 * words, "ks trellis");
+                            for (int r = 0; r < ks_w_runs(S.K); r++)
+                                need_in(S.trellis + at + ks_w_run(S.K, r, lane), S.K == 1 ? 4 : 16, B_TRELLIS + i, 4 * words, "ks trellis run");
+                            const long tile = at / (8 * S.K);
+                            if (tile / S.tc != 2 * q + (lane >> 5) || tile % S.tc != 8 * sg.cg + 4 * h + ((lane & 31) >> 3) ||
+                                at % (8 * S.K) != (lane & 7) * S.K)
+                                fail("ks lane %d decodes another chunk", lane);
+                        }
+                        for (int m = 0; m < mt; m++)
+                            for (int f = 0; f < 2; f++) {
+                                const long c = ks_a_chunk(p0, a.mtt, sg.rt * mt, 0, 0) + (long)(q - p0) * a.mtt * 128 +
+                                               (m * 2 + f) * 64 + lane;
+                                const int row = 32 * (sg.rt * mt + m) + (lane & 31);
+                                const int in8 = 4 * q + 2 * (lane >> 5) + f;
+                                if (c < 0 || c >= chunks || ah[sg.si][c] != row * (W.ic / 8) + in8)
+                                    fail("ks A chunk %ld is not row %d inputs %d", c, row, 8 * in8);
+                            }
+                    }
+                    W.loads++;
+                }
+                if (!split && pair == 0) ks_store_rows(W, shards, a, sg.si, sg.cg, 32 * sg.rt * mt, 32 * mt);
+                W.pieces++;
+            }
+        }
+    }
+    for (size_t i = 0; i < steps.size(); i++)
+        if (steps[i] != 1) fail("ks step %zu decoded %d times", i, steps[i]);
+    for (int quad = 0, seen[1024] = {0}; quad < 8; quad++)
+        for (int c = 0; c < 128; c++) {
+            const int i = ks_slot_in(quad, c);
+            if (i < 0 || i >= 1024 || seen[i]++) fail("ks slot position %d", i);
+        }
+    for (int s = 0; s < a.nrem; s++) {
+        const int g_lo = ks_pair0(a, s) / NP, g_hi = (ks_pair0(a, s + 1) - 1) / NP;
+        for (int g = g_lo; g <= g_hi; g++) {
+            auto it = slot_owner.find(s + g);
+            if (it == slot_owner.end() || it->second != std::make_pair(s, g)) fail("ks finish reads a slot of another piece");
+        }
+        const KsSeg sg = ks_seg(a, a.full * a.G + s);
+        for (int o = 0; o < 4 * mt; o++) {
+            const int row0 = 32 * mt * sg.rt + 8 * o;
+            if (row0 < a.rows) ks_store_rows(W, shards, a, sg.si, sg.cg, row0, 8);
+        }
+    }
+}
+
 }  // namespace
 
 extern "C" {
+
+// The K-split decode-GEMM (exl3_gemm with one shard, exl3_gemm_grouped) of nshards shards that
+// share ic, as exl3r_gemv1.  stats: launches, steps decoded, pieces, slots written.
+int exl3r_gemm_ks(int rows, int ic, int nshards, const int* oc, const int* K, const int* cb, int cus, long long* stats)
+{
+    g_msg.clear();
+    try {
+        if (nshards < 1 || nshards > EXL3_MAX_SHARDS) fail("nshards %d", nshards);
+        KsWorld W;
+        W.rows = rows;
+        W.ic = ic;
+        W.cols = 0;
+        W.ws_bytes = 0;
+        std::vector<GemvShard> shards(nshards);
+        for (int i = 0; i < nshards; i++) {
+            W.sh.push_back(ShardSpec{ic, oc[i], K[i], cb[i]});
+            W.col0.push_back(W.cols);
+            W.cols += oc[i];
+            W.ws_bytes += ks_shard_bytes(rows, ic, oc[i], cus);
+        }
+        W.out.assign((size_t)rows * W.cols, 0);
+        for (int i = 0; i < nshards; i++)
+            shards[i] = GemvShard{fake_ptr<uint32_t>(B_TRELLIS + i), fake_ptr<uint16_t>(B_SUH + i), fake_ptr<uint16_t>(B_SVH + i),
+                                  fake_ptr<uint16_t>(B_C) + W.col0[i], ic, oc[i], K[i], cb[i], W.cols};
+        int launches = 0;
+        const int rc = ks_plan(fake_ptr<uint16_t>(B_X), shards.data(), nshards, rows, fake_ptr<char>(B_WS), W.ws_bytes, "exl3_gemm",
+                               cus, [&](const KsLaunch& L) {
+                                   ks_replay(W, shards.data(), L);
+                                   launches++;
+                                   return EXL3_OK;
+                               });
+        if (rc != EXL3_OK) fail("plan refused: %s", exl3::g_err);
+        for (size_t i = 0; i < W.out.size(); i++)
+            if (W.out[i] != 1) fail("ks output element %zu written %d times", i, W.out[i]);
+        if (stats) {
+            stats[0] = launches;
+            stats[1] = W.loads;
+            stats[2] = W.pieces;
+            stats[3] = W.slot_writes;
+        }
+        return 0;
+    } catch (const Fail& f) {
+        g_msg = f.what;
+        return g_msg.rfind("plan refused", 0) == 0 ? 2 : 1;
+    }
+}
 
 // Message of the last failed replay ("" after a clean one).
 const char* exl3r_message() { return g_msg.c_str(); }
@@ -1206,11 +1472,12 @@ int exl3r_gemv1(int rows, int ic, int nshards, const int* oc, const int* K, cons
 }
 
 
-// The stream-K GEMM for nshards shards sharing ic: mode 0 = exl3_gemm (one shard; up to
-// SK_PREP_MAX_ROWS rows it is the one-shard grouped plan, as gemm_dispatch runs it), 1 =
-// exl3_gemm_grouped; tile height by rows.  Workspaces are sized as the product sizes them for
-// `cus` CUs.  Returns as exl3r_gemv1; stats: launches, K-step loads checked, pieces, slot
-// stores.
+int exl3r_gemm_ks(int rows, int ic, int nshards, const int* oc, const int* K, const int* cb, int cus, long long* stats);
+
+// The prefill GEMM for nshards shards sharing ic: mode 0 = exl3_gemm (one shard), 1 =
+// exl3_gemm_grouped; up to KS_MAX_ROWS rows the K-split decode-GEMM, above the stream-K GEMM.
+// Workspaces are sized as the product sizes them for `cus` CUs.  Returns as exl3r_gemv1;
+// stats: launches, K-step loads checked, pieces, slot stores.
 int exl3r_gemm_sk(int mode, int rows, int ic, int nshards, const int* oc, const int* K, const int* cb, int cus,
                   long long* stats)
 {
@@ -1218,16 +1485,7 @@ int exl3r_gemm_sk(int mode, int rows, int ic, int nshards, const int* oc, const 
     try {
         if (nshards < 1 || nshards > EXL3_MAX_SHARDS || (mode == 0 && nshards != 1) || mode < 0 || mode > 1)
             fail("mode %d, nshards %d", mode, nshards);
-        if (mode == 0 && rows <= SK_PREP_MAX_ROWS) {
-            // exl3_gemm's workspace (its Hadamard output, then counters and slots) is exactly
-            // the one-shard grouped launch's
-            if (gemm_sk_ah_bytes(rows, ic) + sk_single_bytes(rows, oc[0], cus) !=
-                sk_grouped_bytes_bm(gemm_sk_bm(rows), rows, ic, oc[0], cus))
-                fail("exl3_gemm workspace %zu != one-shard grouped workspace %zu",
-                     gemm_sk_ah_bytes(rows, ic) + sk_single_bytes(rows, oc[0], cus),
-                     sk_grouped_bytes_bm(gemm_sk_bm(rows), rows, ic, oc[0], cus));
-            mode = 1;
-        }
+        if (rows <= KS_MAX_ROWS) return exl3r_gemm_ks(rows, ic, nshards, oc, K, cb, cus, stats);
         SkWorld W;
         W.rows = rows;
         W.ic = ic;

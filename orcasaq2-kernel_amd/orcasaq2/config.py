@@ -324,8 +324,9 @@ class Exl3LinearMethod(LinearMethodBase):
         if not xf.is_contiguous():
             xf = xf.contiguous()
         shards = layer.exl3_shards
+        route = _ops._op_route if xf.is_cuda else _ops._fused_route
         if len(shards) > 1 and 0 < rows and (rows <= _ops.GEMM_MAX_ROWS or all(
-                _ops._fused_route(rows, xf.shape[-1], s.oc) for s in shards)):
+                route(rows, xf.shape[-1], s.oc) for s in shards)):
             grouped = torch.ops.orcasaq2.shards_gemv if rows <= GEMV_MAX_ROWS else torch.ops.orcasaq2.shards_gemm
             out = grouped(
                 xf, [s.trellis for s in shards], [s.suh for s in shards], [s.svh for s in shards],

@@ -13,13 +13,12 @@ Dispatch on the number of activation rows (reference: orcasaq2/ops.py:25, 46-59)
                           whose add completes it); rows 5..16, and 2..4-row shards too large for
                           that kernel's tables: the same decode on 4 x 2-tile units, one MFMA
                           serving all rows; output Hadamard and svh at the end;
-  * 16 < rows <= GEMM_MAX_ROWS
-                          fused decode-GEMM (exl3_gemm): Hadamard pass over x, then stream-K
-                          tiles decoded straight into MFMA operands, output Hadamard in the
-                          epilogue; a fused layer's shards together (shards_gemm) -- except a
-                          single shard with 4096 <= ic < 8192 above 64 rows where the
-                          reconstruct branch measured faster (_fused_gemm_faster);
-  * rows > GEMM_MAX_ROWS  the reference's reconstruct branch: had_r_128(x, suh), dense W_q
+  * 16 < rows <= SPLIT_MAX_ROWS
+                          fused decode-GEMM (exl3_gemm): set-up of x in fragment order, the
+                          K-split decode into MFMA operands, a finishing launch; a fused layer's
+                          shards together (shards_gemm).  A row knob set lower is the
+                          reference's hard switch to the reconstruct branch;
+  * above                 the reference's reconstruct branch: had_r_128(x, suh), dense W_q
                           (decoded transposed, (oc, ic)) into a scratch freed on exit, library
                           fp16 transposed-B GEMM, had_r_128(y, svh) -- except, while the row
                           knob is at its default, 8192+ inputs up to WIDE_FUSED_MAX_ROWS rows
@@ -45,6 +44,7 @@ from . import _native
 # reference.
 GEMM_MAX_ROWS = int(os.environ.get("ORCA_EXL3_GEMM_MAX_ROWS", "144"))
 GEMM_MAX_ROWS_SET = "ORCA_EXL3_GEMM_MAX_ROWS" in os.environ
+SPLIT_MAX_ROWS = 512                 # every shard: the K-split decode-GEMM up to here
 WIDE_FUSED_MAX_ROWS = 2560           # 8192+ inputs: fused up to here
 WIDE_OUT_FUSED_ROWS = (1536, 3072)   # 4096..8191 inputs, oc >= 2 ic: fused in (lo, hi] too
 GEMV_MAX_ROWS = _native.GEMV_MAX_ROWS
@@ -92,6 +92,18 @@ def _fused_route(rows: int, ic: int, oc: int) -> bool:
     return not GEMM_MAX_ROWS_SET and ic >= 4096 and _fused_gemm_faster(rows, ic, oc)
 
 
+def _op_route(rows: int, ic: int, oc: int) -> bool:
+    """Whether the ops take the fused path for rows > GEMV_MAX_ROWS.  Up to SPLIT_MAX_ROWS rows the
+    library runs the K-split decode-GEMM, measured faster than the reconstruct branch on every
+    shape there (us, fused / branch: 5120 -> 6144 at 144 rows 37 / 53, 256: 39 / 73, 384: 48 / 64;
+    5120 -> 17408 at 144 rows 78 / 95, 256: 81 / 109, 384: 105 / 118; 17408 -> 5120 at 384 rows
+    102 / 183), unless the row knob is set below; above, the stream-K kernel where it measured
+    faster (_fused_route)."""
+    if rows <= SPLIT_MAX_ROWS:
+        return rows <= GEMM_MAX_ROWS or not GEMM_MAX_ROWS_SET
+    return _fused_route(rows, ic, oc)
+
+
 def _shard_gemm_impl(x: Tensor, trellis: Tensor, suh: Tensor, svh: Tensor, oc: int, k: float,
                      mcg: bool, mul1: bool) -> Tensor:
     cb = _native.codebook_id(mcg, mul1)
@@ -102,7 +114,7 @@ def _shard_gemm_impl(x: Tensor, trellis: Tensor, suh: Tensor, svh: Tensor, oc: i
         return x.new_empty((0, oc), dtype=torch.half)
     if rows <= GEMV_MAX_ROWS:
         return _native.gemv(x, trellis, suh, svh, k, cb)
-    if _fused_route(rows, ic, oc):
+    if _op_route(rows, ic, oc):
         return _native.gemm(x, trellis, suh, svh, k, cb)
     return _reconstruct_branch(x, trellis, suh, svh, k, cb)
 
