@@ -93,6 +93,17 @@ int exl3_had_r_128(const void* in, void* out, const void* pre, const void* post,
                    long rows, int cols, void* stream);
 
 /*
+ * exl3_had_r_128 with typed input and output (EXL3_IO_F16 or EXL3_IO_BF16) and an output row
+ * stride of ld_out elements (even, >= cols), so that a shard's result can land in its columns of
+ * a concatenated output.  bfloat16 inputs are rounded to fp16 first; bfloat16 outputs are the
+ * fp16 result rounded once more.
+ */
+#define EXL3_IO_F16 0
+#define EXL3_IO_BF16 1
+int exl3_had_r_128_io(const void* in, int in_dtype, void* out, int out_dtype, long ld_out, const void* pre,
+                      const void* post, float scale, long rows, int cols, void* stream);
+
+/*
  * Fused decode-GEMV, 1 <= rows <= 16:
  *   C (rows, oc) = fp16( H( fp16(H(A * suh)) . W_q ) * svh ),  A (rows, ic) fp16.
  * Replaces ext.exl3_gemm(A, trellis, C, suh, A_had, svh, -1, mcg, mul1, 0)
@@ -135,6 +146,14 @@ int exl3_gemv_grouped(const void* A, const exl3_shard_t* shards, int nshards, vo
                       size_t ws_bytes, int rows, int ic, void* stream);
 
 /*
+ * exl3_gemv_grouped with A and every C of type io_dtype (EXL3_IO_F16: as exl3_gemv_grouped).
+ * EXL3_IO_BF16 gives what rounding A to fp16 and the fp16 outputs to bfloat16 around the call
+ * gives, inside the kernels' loads and stores.
+ */
+int exl3_gemv_grouped_io(const void* A, const exl3_shard_t* shards, int nshards, int io_dtype, void* workspace,
+                         size_t ws_bytes, int rows, int ic, void* stream);
+
+/*
  * exl3_gemv_grouped without a workspace argument: it allocates nothing (no hipMalloc, no
  * library allocation), for callers that cannot allocate -- code under HIP-graph capture,
  * serving loops that forbid device allocation.  No counterpart in the reference.
@@ -174,6 +193,10 @@ int exl3_gemm(const void* A, const void* trellis, void* C, const void* suh, cons
 size_t exl3_gemm_grouped_workspace_bytes(const exl3_shard_t* shards, int nshards, int rows, int ic);
 int exl3_gemm_grouped(const void* A, const exl3_shard_t* shards, int nshards, void* workspace,
                       size_t ws_bytes, int rows, int ic, void* stream);
+
+/* exl3_gemm_grouped with A and every C of type io_dtype (see exl3_gemv_grouped_io). */
+int exl3_gemm_grouped_io(const void* A, const exl3_shard_t* shards, int nshards, int io_dtype, void* workspace,
+                         size_t ws_bytes, int rows, int ic, void* stream);
 
 /*
  * int8 embedding gather: out[n, :] = dtype(table[ids[n], :]) * scales[ids[n]], computed

@@ -84,7 +84,7 @@ extern "C" {
 
 const char* exl3_last_error(void) { return g_err; }
 
-int exl3_abi_version(void) { return 7; }
+int exl3_abi_version(void) { return 8; }
 
 int exl3_stream_capture_id(void* stream, unsigned long long* id)
 {
@@ -132,16 +132,24 @@ int exl3_reconstruct_t(void* Wt, const void* trellis, int ic, int oc, int K, int
 int exl3_had_r_128(const void* in, void* out, const void* pre, const void* post, float scale, long rows, int cols,
                    void* stream)
 {
+    return exl3_had_r_128_io(in, EXL3_IO_F16, out, EXL3_IO_F16, cols, pre, post, scale, rows, cols, stream);
+}
+
+int exl3_had_r_128_io(const void* in, int in_dtype, void* out, int out_dtype, long ld_out, const void* pre,
+                      const void* post, float scale, long rows, int cols, void* stream)
+{
     g_err[0] = 0;
     if (!in || !out) return set_error(EXL3_ERR_ARG, "exl3_had_r_128: null in/out");
     if (rows < 0 || cols <= 0 || cols % 128)
         return set_error(EXL3_ERR_ARG, "exl3_had_r_128: rows=%ld, cols=%d (cols must be a multiple of 128)", rows,
                          cols);
+    if (in_dtype < 0 || in_dtype > EXL3_IO_BF16 || out_dtype < 0 || out_dtype > EXL3_IO_BF16 || ld_out < cols || ld_out % 2)
+        return set_error(EXL3_ERR_ARG, "exl3_had_r_128: dtypes %d, %d, ld_out=%ld (even, >= cols)", in_dtype, out_dtype, ld_out);
     if (!aligned(in, 4) || !aligned(out, 4) || (pre && !aligned(pre, 4)) || (post && !aligned(post, 4)))
         return set_error(EXL3_ERR_ARG, "exl3_had_r_128: pointers must be 4-byte aligned");
     return had_dispatch(static_cast<const uint16_t*>(in), static_cast<uint16_t*>(out),
                         static_cast<const uint16_t*>(pre), static_cast<const uint16_t*>(post), scale, rows, cols,
-                        static_cast<hipStream_t>(stream));
+                        static_cast<hipStream_t>(stream), nullptr, 0, in_dtype, out_dtype, ld_out);
 }
 
 size_t exl3_gemv_workspace_bytes(int rows, int ic, int oc)
@@ -164,7 +172,15 @@ size_t exl3_gemv_grouped_workspace_bytes(const exl3_shard_t* shards, int nshards
 int exl3_gemv_grouped(const void* A, const exl3_shard_t* shards, int nshards, void* workspace, size_t ws_bytes,
                       int rows, int ic, void* stream)
 {
+    return exl3_gemv_grouped_io(A, shards, nshards, EXL3_IO_F16, workspace, ws_bytes, rows, ic, stream);
+}
+
+int exl3_gemv_grouped_io(const void* A, const exl3_shard_t* shards, int nshards, int io_dtype, void* workspace,
+                         size_t ws_bytes, int rows, int ic, void* stream)
+{
     g_err[0] = 0;
+    const int bf = io_dtype;
+    if (bf != EXL3_IO_F16 && bf != EXL3_IO_BF16) return set_error(EXL3_ERR_ARG, "exl3_gemv: io dtype %d", io_dtype);
     if (!A || !shards || nshards < 1 || nshards > EXL3_MAX_SHARDS)
         return set_error(EXL3_ERR_ARG, "exl3_gemv: need A and 1..%d shards (got %d)", EXL3_MAX_SHARDS, nshards);
     if (!workspace) return set_error(EXL3_ERR_ARG, "exl3_gemv: null workspace");
@@ -179,7 +195,7 @@ int exl3_gemv_grouped(const void* A, const exl3_shard_t* shards, int nshards, vo
             return set_error(EXL3_ERR_ARG, "exl3_gemv: shard %d: C must be 4-byte aligned with even ldc >= oc", i);
         d[i] = GemvShard{static_cast<const uint32_t*>(s.trellis), static_cast<const uint16_t*>(s.suh),
                          static_cast<const uint16_t*>(s.svh), static_cast<uint16_t*>(s.C), ic, s.oc, s.K,
-                         s.codebook, s.ldc};
+                         s.codebook, s.ldc, bf};
     }
     return gemv_dispatch(static_cast<const uint16_t*>(A), d, nshards, rows, workspace, ws_bytes,
                          static_cast<hipStream_t>(stream));
@@ -228,7 +244,15 @@ size_t exl3_gemm_grouped_workspace_bytes(const exl3_shard_t* shards, int nshards
 int exl3_gemm_grouped(const void* A, const exl3_shard_t* shards, int nshards, void* workspace, size_t ws_bytes,
                       int rows, int ic, void* stream)
 {
+    return exl3_gemm_grouped_io(A, shards, nshards, EXL3_IO_F16, workspace, ws_bytes, rows, ic, stream);
+}
+
+int exl3_gemm_grouped_io(const void* A, const exl3_shard_t* shards, int nshards, int io_dtype, void* workspace,
+                         size_t ws_bytes, int rows, int ic, void* stream)
+{
     g_err[0] = 0;
+    const int bf = io_dtype;
+    if (bf != EXL3_IO_F16 && bf != EXL3_IO_BF16) return set_error(EXL3_ERR_ARG, "exl3_gemm_grouped: io dtype %d", io_dtype);
     if (!A || !shards || nshards < 1 || nshards > EXL3_MAX_SHARDS)
         return set_error(EXL3_ERR_ARG, "exl3_gemm_grouped: need A and 1..%d shards (got %d)", EXL3_MAX_SHARDS,
                          nshards);
@@ -247,7 +271,7 @@ int exl3_gemm_grouped(const void* A, const exl3_shard_t* shards, int nshards, vo
                              i);
         d[i] = GemvShard{static_cast<const uint32_t*>(s.trellis), static_cast<const uint16_t*>(s.suh),
                          static_cast<const uint16_t*>(s.svh), static_cast<uint16_t*>(s.C), ic, s.oc, s.K,
-                         s.codebook, s.ldc};
+                         s.codebook, s.ldc, bf};
     }
     if (ws_bytes < need)
         return set_error(EXL3_ERR_WORKSPACE, "exl3_gemm_grouped: workspace of %zu bytes, %zu needed", ws_bytes, need);

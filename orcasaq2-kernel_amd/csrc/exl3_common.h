@@ -423,6 +423,33 @@ __device__ __forceinline__ void chunk_prev_dpp(uint32_t (&w)[K + 1], bool first_
     w[0] = first_lane ? r9 : r1;
 }
 
+// ---------------------------------------------------------------- activation and output types
+//
+// A caller's activations and outputs are fp16, or (bf) bfloat16.  bfloat16 activations are rounded
+// to fp16 and outputs are rounded to fp16 and then to bfloat16, each to nearest even: the values
+// that separate conversions around an fp16 call give, without their passes over memory.
+
+// Two activations (one 32-bit word) as fp16 bits.
+__device__ __forceinline__ uint32_t act_pair(uint32_t w, int bf)
+{
+    if (!bf) return w;
+    const float lo = __builtin_bit_cast(float, w << 16), hi = __builtin_bit_cast(float, w & 0xffff0000u);
+    return (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)lo) | ((uint32_t)__builtin_bit_cast(uint16_t, (_Float16)hi) << 16);
+}
+
+// An output rounded to fp16, as the bits stored.
+__device__ __forceinline__ uint32_t out_half(_Float16 h, int bf)
+{
+    if (!bf) return __builtin_bit_cast(uint16_t, h);
+    const float f = (float)h;
+    const uint32_t u = __builtin_bit_cast(uint32_t, f);
+    return f != f ? 0x7fc0u : (u + 0x7fffu + ((u >> 16) & 1u)) >> 16;
+}
+__device__ __forceinline__ uint32_t out_pair(float v0, float v1, int bf)
+{
+    return out_half((_Float16)v0, bf) | (out_half((_Float16)v1, bf) << 16);
+}
+
 // ---------------------------------------------------------------- wave helpers
 
 // In-wave normalised Walsh-Hadamard of one 128-vector held as v0 = x[2l], v1 = x[2l+1]

@@ -24,9 +24,11 @@ int device_cus();
 int reconstruct_dispatch(uint16_t* W, const uint32_t* trellis, int ic, int oc, int K, int cb, bool transposed,
                          hipStream_t stream);
 // zero / nzero: 32-bit words the first workgroup sets to 0 (a following launch's counters:
-// one launch fewer than a fill kernel of their own), or none.
+// one launch fewer than a fill kernel of their own), or none.  in_bf / out_bf: bfloat16 instead of
+// fp16; ld_out: output row stride in elements (0: cols).
 int had_dispatch(const uint16_t* in, uint16_t* out, const uint16_t* pre, const uint16_t* post,
-                 float scale, long rows, int cols, hipStream_t stream, uint32_t* zero = nullptr, int nzero = 0);
+                 float scale, long rows, int cols, hipStream_t stream, uint32_t* zero = nullptr, int nzero = 0,
+                 int in_bf = 0, int out_bf = 0, long ld_out = 0);
 
 struct GemvShard {
     const uint32_t* trellis;
@@ -35,6 +37,7 @@ struct GemvShard {
     uint16_t* C;       // (rows, ldc) fp16; this shard writes columns [0, oc)
     int ic, oc, K, cb;
     long ldc;
+    int bf = 0;        // 1: activations and outputs are bfloat16
 };
 
 // A GEMV workspace: a reserved 16 KiB head (no kernel reads or writes it), then the
@@ -69,10 +72,7 @@ size_t gemm_ks_shard_bytes(int rows, int ic, int oc);
 int gemm_ks_dispatch(const uint16_t* A, const GemvShard* shards, int nshards, int rows, char* ws, size_t ws_bytes,
                      hipStream_t stream, const char* what);
 int gemm_sk_cus();
-// The launch's tile counters, the first sk_ntiles(rows, oc) words of ws, must be 0 when it
-// starts (exl3_gemm's Hadamard pass clears them).
-int gemm_sk_dispatch(const uint16_t* Ah, const uint32_t* trellis, uint16_t* C, const uint16_t* svh, char* ws,
-                     size_t ws_bytes, int rows, int ic, int oc, int K, int cb, hipStream_t stream);
+int gemm_sk_dispatch(const uint16_t* A, const GemvShard& d, char* ws, size_t ws_bytes, int rows, hipStream_t stream);
 int embed_dispatch(const int8_t* table, const void* scales, int scale_dtype, const int64_t* ids,
                    void* out, long n_ids, int vocab, int dim, hipStream_t stream);
 

@@ -29,17 +29,8 @@ int gemm_dispatch(const uint16_t* A, const uint32_t* trellis, uint16_t* C, const
     if (ws_bytes < need)
         return set_error(EXL3_ERR_WORKSPACE, "exl3_gemm: workspace of %zu bytes, %zu needed", ws_bytes, need);
     if (K < 1 || K > 8) return set_error(EXL3_ERR_ARG, "exl3_gemm: K=%d is not in 1..8", K);
-    if (rows <= KS_MAX_ROWS) {
-        const GemvShard d{trellis, suh, svh, C, ic, oc, K, cb, (long)oc};
-        return gemm_ks_dispatch(A, &d, 1, rows, static_cast<char*>(workspace), ws_bytes, stream, "exl3_gemm");
-    }
-    uint16_t* Ah = static_cast<uint16_t*>(workspace);
-    const size_t ah = gemm_sk_ah_bytes(rows, ic);
-    char* const sk_ws = static_cast<char*>(workspace) + ah;   // tile counters first, then slots
-    int rc = had_dispatch(A, Ah, suh, nullptr, 1.0f, rows, ic, stream, reinterpret_cast<uint32_t*>(sk_ws),
-                          sk_ntiles(rows, oc));
-    if (rc != EXL3_OK) return rc;
-    return gemm_sk_dispatch(Ah, trellis, C, svh, sk_ws, ws_bytes - ah, rows, ic, oc, K, cb, stream);
+    const GemvShard d{trellis, suh, svh, C, ic, oc, K, cb, (long)oc};
+    return gemm_grouped_dispatch(A, &d, 1, rows, static_cast<char*>(workspace), ws_bytes, stream, "exl3_gemm");
 }
 
 }  // namespace exl3

@@ -49,7 +49,7 @@ __global__ __launch_bounds__(512) void ks_prep_kernel(const KsPrepArgs p)
         __builtin_memcpy(&x, p.A + (long)grow * p.ic + b * 128 + 8 * l16, 16);
         __builtin_memcpy(&sg, p.suh[s] + b * 128 + 8 * l16, 16);
         float v[8], f[8];
-        had_unpack(x, v);
+        had_unpack(uint4{act_pair(x.x, p.bf), act_pair(x.y, p.bf), act_pair(x.z, p.bf), act_pair(x.w, p.bf)}, v);
         had_unpack(sg, f);
 #pragma unroll
         for (int i = 0; i < 8; i++) v[i] *= f[i];
@@ -289,7 +289,7 @@ __device__ __forceinline__ void ks_steps(KsAcc<MT>& acc, const KsShard& S, const
 // Output rows: the fp32 row staged at `st` (128 outputs, lane l the pair 2 l, 2 l + 1) through
 // the output Hadamard and svh.
 template <int N>
-__device__ __forceinline__ void ks_rows_out(const float* st, int row0, int rows, const KsShard& S, int cg, int lane)
+__device__ __forceinline__ void ks_rows_out(const float* st, int row0, int rows, const KsShard& S, int cg, int bf, int lane)
 {
     const uint32_t sv = reinterpret_cast<const uint32_t*>(S.svh + cg * 128)[lane];
     const float s0 = (float)__builtin_bit_cast(_Float16, (uint16_t)(sv & 0xffffu));
@@ -306,8 +306,7 @@ __device__ __forceinline__ void ks_rows_out(const float* st, int row0, int rows,
     for (int r = 0; r < N; r++)
         if (row0 + r < rows)
             reinterpret_cast<uint32_t*>(S.C + (long)(row0 + r) * S.ldc + cg * 128)[lane] =
-                (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)(v0[r] * s0)) |
-                ((uint32_t)__builtin_bit_cast(uint16_t, (_Float16)(v1[r] * s1)) << 16);
+                out_pair(v0[r] * s0, v1[r] * s1, bf);
 }
 
 // The waves' accumulators of 32-row block m to LDS, by column position.
@@ -425,7 +424,7 @@ void gemm_ks_kernel(const KsArgs a)
                 }
                 ks_barrier();
                 constexpr int NR = 32 / (2 * NP);
-                ks_rows_out<NR>(red + wave * NR * KS_LDC, 32 * (sg.rt * MT + m) + wave * NR, a.rows, S, sg.cg, lane);
+                ks_rows_out<NR>(red + wave * NR * KS_LDC, 32 * (sg.rt * MT + m) + wave * NR, a.rows, S, sg.cg, a.bf, lane);
                 ks_barrier();
             }
         }
@@ -464,7 +463,7 @@ __global__ __launch_bounds__(256) void ks_finish_kernel(const KsArgs a, int mt)
     p[3 * KS_LDC] = v.w;
     __syncthreads();
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    ks_rows_out<2>(st + 2 * wave * KS_LDC, row0 + 2 * wave, a.rows, S, sg.cg, tid & 63);
+    ks_rows_out<2>(st + 2 * wave * KS_LDC, row0 + 2 * wave, a.rows, S, sg.cg, a.bf, tid & 63);
 }
 
 // ---------------------------------------------------------------- host side

@@ -85,6 +85,7 @@ struct KsShard {
 struct KsArgs {
     float* slots;              // (nrem + G) x MT x 32 x 128 fp32 partial sums
     int rows, P, mtt;          // mtt: 32-row tiles in all (row tiles x MT)
+    int bf;                    // outputs are bfloat16
     int nrt, nshards, G, full, nrem;
     // the split segments' pairs and steps: the first pextra of them have pbase + 1 pairs, the
     // others pbase; among c pairs the first P % c have P / c + 1 steps, the others P / c
@@ -97,6 +98,7 @@ struct KsArgs {
 struct KsPrepArgs {
     const uint16_t* A;
     int rows, ic, nsh, nblk, mtt;
+    int bf;                    // A is bfloat16
     const uint16_t* suh[KS_MAXSH];
     uint16_t* Ah[KS_MAXSH];
 };
@@ -243,6 +245,7 @@ int ks_plan(const uint16_t* A, const GemvShard* shards, int nshards, int rows, c
         KsArgs a = {};
         KsPrepArgs p = {};
         a.rows = p.rows = rows;
+        a.bf = p.bf = shards[i].bf;
         a.P = ic / KS_PIN;
         a.mtt = p.mtt = t.nrt * t.mt;
         p.A = A;

@@ -43,7 +43,7 @@ __global__ __launch_bounds__(256) void sk_prep_kernel(const SkPrepArgs a)
     int s, r, b;
     sk_prep_wave(a, w, s, r, b);
     const long off = sk_prep_elem(a, r, b);
-    const uint32_t xw = reinterpret_cast<const uint32_t*>(a.A + off)[lane];
+    const uint32_t xw = act_pair(reinterpret_cast<const uint32_t*>(a.A + off)[lane], a.bf);
     const uint32_t sw = reinterpret_cast<const uint32_t*>(a.suh[s] + b * 128)[lane];
     float v0 = (float)__builtin_bit_cast(_Float16, (uint16_t)(xw & 0xffffu)) *
                (float)__builtin_bit_cast(_Float16, (uint16_t)(sw & 0xffffu));
@@ -203,7 +203,7 @@ __device__ __forceinline__ void sk_finish_piece(const SkArgs& a, const SkPiece& 
         // in registers: the LDS barriers below clobber memory, which would reload these
         uint16_t* const Cp = S.C;
         const long ldc = S.ldc;
-        const int rows = a.rows;
+        const int rows = a.rows, bf = a.bf;
         // svh pair of this lane in the 128-output block starting at tile column ob, read
         // once per block: the fp16 output stores could alias it, so a load inside the
         // row loop would be repeated (a round trip per row)
@@ -229,8 +229,7 @@ __device__ __forceinline__ void sk_finish_piece(const SkArgs& a, const SkPiece& 
             // ob: tile column of the 128-output block's first output; v0, v1 transformed
             if (ob < tc && row < rows) {
                 const float sv0 = sv.s0, sv1 = sv.s1;
-                const uint32_t o = (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)(v0 * sv0)) |
-                                   ((uint32_t)__builtin_bit_cast(uint16_t, (_Float16)(v1 * sv1)) << 16);
+                const uint32_t o = out_pair(v0 * sv0, v1 * sv1, bf);
                 reinterpret_cast<uint32_t*>(Cp + (long)row * ldc + ob * 16)[lane] = o;
             }
         };
@@ -786,10 +785,20 @@ static int sk_emit(const SkLaunch& L, const char* what, hipStream_t stream)
     return check_launch(what);
 }
 
-int gemm_sk_dispatch(const uint16_t* Ah, const uint32_t* trellis, uint16_t* C, const uint16_t* svh, char* ws,
-                     size_t ws_bytes, int rows, int ic, int oc, int K, int cb, hipStream_t stream)
+// One shard above KS_MAX_ROWS rows: the 16-byte-lane Hadamard pass into the head of the workspace
+// (its first workgroup clears the launch's tile counters), then the stream-K launch.  The
+// workspace is the one-shard grouped launch's.
+int gemm_sk_dispatch(const uint16_t* A, const GemvShard& d, char* ws, size_t ws_bytes, int rows, hipStream_t stream)
 {
-    return sk_plan_single(Ah, trellis, C, svh, ws, ws_bytes, rows, ic, oc, K, cb, gemm_sk_cus(),
+    const size_t ah = gemm_sk_ah_bytes(rows, d.ic);
+    if (ws_bytes < ah + gemm_sk_slot_bytes(rows, d.oc))
+        return set_error(EXL3_ERR_WORKSPACE, "exl3_gemm: workspace of %zu bytes, %zu needed", ws_bytes,
+                         ah + gemm_sk_slot_bytes(rows, d.oc));
+    uint16_t* Ah = reinterpret_cast<uint16_t*>(ws);
+    const int rc = had_dispatch(A, Ah, d.suh, nullptr, 1.0f, rows, d.ic, stream, reinterpret_cast<uint32_t*>(ws + ah),
+                                sk_ntiles(rows, d.oc), d.bf);
+    if (rc != EXL3_OK) return rc;
+    return sk_plan_single(Ah, d, ws + ah, ws_bytes - ah, rows, gemm_sk_cus(),
                           [&](const SkLaunch& L) { return sk_emit(L, "exl3_gemm (stream-K)", stream); });
 }
 
@@ -807,6 +816,7 @@ int gemm_grouped_dispatch(const uint16_t* A, const GemvShard* shards, int nshard
                           size_t ws_bytes, hipStream_t stream, const char* what)
 {
     if (rows <= KS_MAX_ROWS) return gemm_ks_dispatch(A, shards, nshards, rows, ws, ws_bytes, stream, what);
+    if (nshards == 1) return gemm_sk_dispatch(A, shards[0], ws, ws_bytes, rows, stream);
     switch (gemm_sk_bm(rows)) {
     case 32: return sk_grouped_dispatch<32>(A, shards, nshards, rows, ws, ws_bytes, what, stream);
     case 48: return sk_grouped_dispatch<48>(A, shards, nshards, rows, ws, ws_bytes, what, stream);

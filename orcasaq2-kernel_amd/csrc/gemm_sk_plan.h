@@ -66,6 +66,7 @@ struct SkArgs {
     uint32_t* counters;        // one per tile, zeroed before the launch
     float* slots;              // (tiles + G) x SK_WAVES x acc x 64 fp32
     int rows, ic, nks, ntiles, nshards;
+    int bf;                    // outputs are bfloat16
     int q, r;                  // K-steps per workgroup: q + (g < r)
     SkShard sh[SK_MAXSH];
 };
@@ -76,6 +77,7 @@ struct SkArgs {
 struct SkPrepArgs {
     const uint16_t* A;
     int rows, ic, nsh, nblk;
+    int bf;                    // A is bfloat16
     const uint16_t* suh[SK_MAXSH];
     uint16_t* Ah[SK_MAXSH];
     uint32_t* counters;
@@ -378,30 +380,31 @@ inline int sk_ntiles(int rows, int oc)
 // exl3_gemm's stream-K launch over one shard (Ah already transformed; its tile counters
 // cleared by the same Hadamard pass).
 template <class Emit>
-int sk_plan_single(const uint16_t* Ah, const uint32_t* trellis, uint16_t* C, const uint16_t* svh, char* ws,
-                   size_t ws_bytes, int rows, int ic, int oc, int K, int cb, int cus, Emit&& emit)
+int sk_plan_single(const uint16_t* Ah, const GemvShard& d, char* ws, size_t ws_bytes, int rows, int cus, Emit&& emit)
 {
+    const int ic = d.ic, oc = d.oc;
     SkArgs a = {};
     a.rows = rows;
+    a.bf = d.bf;
     a.ic = ic;
     a.nks = ic / SK_KS;
     a.nshards = 1;
     SkShard& s = a.sh[0];
     s.Ah = Ah;
-    s.trellis = trellis;
-    s.svh = svh;
-    s.C = C;
-    s.ldc = oc;
+    s.trellis = d.trellis;
+    s.svh = d.svh;
+    s.C = d.C;
+    s.ldc = d.ldc;
     s.oc = oc;
     s.ntn = sk_ntn(oc);
     s.tbeg = 0;
-    s.K = K;
+    s.K = d.K;
     const int bm = gemm_sk_bm(rows);
     a.ntiles = sk_ntiles(rows, oc);
     SkLaunch L = {};
     L.BM = bm;
-    L.K = K;
-    L.cb = cb;
+    L.K = d.K;
+    L.cb = d.cb;
     L.args = &a;
     const char* what = "exl3_gemm (stream-K)";
     int rc;
@@ -435,6 +438,7 @@ int sk_plan_grouped(const uint16_t* A, const GemvShard* shards, int nshards, int
         SkArgs a = {};
         SkPrepArgs p = {};
         a.rows = p.rows = rows;
+        a.bf = p.bf = shards[i].bf;
         a.ic = p.ic = ic;
         a.nks = ic / SK_KS;
         p.A = A;

@@ -153,15 +153,15 @@ __device__ __forceinline__ void g1_acc_add(const G1Group& a, const G1Shard* sht,
     if (!f0 && !f1) return;
     const unsigned long long all = (unsigned long long)n << G1_FX_CBIT;
     constexpr double unit = 1.0 / (double)(1 << G1_FX_FRAC);
-    const uint16_t h0 = __builtin_bit_cast(uint16_t, (_Float16)(float)((double)(long long)(o0 + m0 - all) * unit));
-    const uint16_t h1 = __builtin_bit_cast(uint16_t, (_Float16)(float)((double)(long long)(o1 + m1 - all) * unit));
+    const uint32_t h0 = out_half((_Float16)(float)((double)(long long)(o0 + m0 - all) * unit), a.bf);
+    const uint32_t h1 = out_half((_Float16)(float)((double)(long long)(o1 + m1 - all) * unit), a.bf);
     uint16_t* c = e.C + r * e.ldc + cg * 128 + 2 * lane;
     if (f0 && f1) {
-        *reinterpret_cast<uint32_t*>(c) = (uint32_t)h0 | ((uint32_t)h1 << 16);
+        *reinterpret_cast<uint32_t*>(c) = h0 | (h1 << 16);
     } else if (f0) {
-        c[0] = h0;
+        c[0] = (uint16_t)h0;
     } else {
-        c[1] = h1;
+        c[1] = (uint16_t)h1;
     }
     if (f0) __hip_atomic_store(p, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (f1) __hip_atomic_store(p + 1, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -260,7 +260,8 @@ __device__ __forceinline__ void g1_body(const G1Group& a, const G1Shard* sht, co
 #pragma unroll
         for (int j = 0; j < G1_TBATCH; j++) {
             if (tb[j].t < ntask) {
-                float v0 = g1_lo(xw[j]) * g1_lo(sw[j]), v1 = g1_hi(xw[j]) * g1_hi(sw[j]);
+                const uint32_t xa = act_pair(xw[j], a.bf);
+                float v0 = g1_lo(xa) * g1_lo(sw[j]), v1 = g1_hi(xa) * g1_hi(sw[j]);
                 wave_fwht128(v0, v1, fs);
                 *reinterpret_cast<uint2*>(act + g1_act_word(tb[j].i, lane, nr, tb[j].r)) = uint2{g1_dup(v0), g1_dup(v1)};
             }
@@ -345,9 +346,7 @@ __device__ __forceinline__ void g1_body(const G1Group& a, const G1Shard* sht, co
         wave_fwht128(v0, v1);
         v0 *= g1_lo(sv);
         v1 *= g1_hi(sv);
-        const uint32_t out = (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)v0) |
-                             ((uint32_t)__builtin_bit_cast(uint16_t, (_Float16)v1) << 16);
-        reinterpret_cast<uint32_t*>(sh(s).C + r * sh(s).ldc + cg * 128)[lane] = out;
+        reinterpret_cast<uint32_t*>(sh(s).C + r * sh(s).ldc + cg * 128)[lane] = out_pair(v0, v1, a.bf);
     };
     // (segment, activation row) tasks shared out over the waves
     for (int t = wave; t < w.nseg * nr; t += G1_NW) {
@@ -465,7 +464,7 @@ __device__ __forceinline__ void g1_finish_body(const G1Group& a, const G1Shard* 
         v0 *= g1_lo(sv);
         v1 *= g1_hi(sv);
         reinterpret_cast<uint32_t*>(sh(s).C + r * sh(s).ldc + cg * 128)[lane] =
-            (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)v0) | ((uint32_t)__builtin_bit_cast(uint16_t, (_Float16)v1) << 16);
+            out_pair(v0, v1, a.bf);
     }
 }
 

@@ -256,7 +256,7 @@ __device__ __forceinline__ void g16_finish_body(const G1Group& a, const G16Shard
         v0 *= (float)__builtin_bit_cast(_Float16, (uint16_t)(sv & 0xffffu));
         v1 *= (float)__builtin_bit_cast(_Float16, (uint16_t)(sv >> 16));
         reinterpret_cast<uint32_t*>(e.C + r * e.ldc + cg * 128)[lane] =
-            (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)v0) | ((uint32_t)__builtin_bit_cast(uint16_t, (_Float16)v1) << 16);
+            out_pair(v0, v1, a.bf);
     }
 }
 
@@ -293,7 +293,7 @@ __global__ __launch_bounds__(G16_PREP_LANES) void gemv16_prep_kernel(const G16Pr
 #pragma unroll
     for (int j = 0; j < 4; j++) {
         const int r = wv + 4 * j;
-        const uint32_t xw = r < p.rows ? reinterpret_cast<const uint32_t*>(p.A + (long)r * p.ic + b * 128)[lane] : 0u;
+        const uint32_t xw = r < p.rows ? act_pair(reinterpret_cast<const uint32_t*>(p.A + (long)r * p.ic + b * 128)[lane], p.bf) : 0u;
         v0[j] = (float)__builtin_bit_cast(_Float16, (uint16_t)(xw & 0xffffu)) * s0;
         v1[j] = (float)__builtin_bit_cast(_Float16, (uint16_t)(xw >> 16)) * s1;
     }

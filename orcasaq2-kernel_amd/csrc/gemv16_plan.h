@@ -271,6 +271,7 @@ inline size_t g16_shard_bytes(int ic, int oc)
 struct G16Prep {
     const uint16_t* A;
     int rows, ic, nsh, nblk;
+    int bf;                    // A is bfloat16
     const uint16_t* suh[EXL3_MAX_SHARDS];
     uint32_t* ah[EXL3_MAX_SHARDS];
 };
@@ -313,6 +314,7 @@ inline long g16_group(G1Group& grp, G16Shard* tab, const GemvShard* shards, cons
 {
     grp = G1Group{};
     grp.nrows = rows;
+    grp.bf = shards[idx[0]].bf;
     grp.ntr = nq;
     grp.nshards = n;
     long U = 0;
@@ -410,6 +412,7 @@ int g16_plan(const uint16_t* A, const GemvShard* shards, int nshards, int rows, 
     prep = G16Prep{};
     prep.A = A;
     prep.rows = rows;
+    prep.bf = shards[0].bf;
     prep.ic = ic;
     prep.nsh = nshards;
     prep.nblk = ic / 128;

@@ -71,6 +71,7 @@ G1_HD int g1_div(int x, G1Div d)
 struct G1Group {
     const uint16_t* x;         // (nrows, ic) fp16
     int nrows;                 // activation rows, 1 .. R of the kernel
+    int bf;                    // activations and outputs are bfloat16
     float* slots;              // (G + segments) x R x 128 fp32 partials of split segments (acc null)
     unsigned long long* acc;   // segments x R x 128 accumulator words of split segments, or null
     int U, G, ntr, nshards, nsegs;
@@ -542,6 +543,7 @@ inline long g1_group(G1Group& grp, G1Shard* tab, const GemvShard* shards, const 
     grp = G1Group{};
     grp.x = A;
     grp.nrows = rows;
+    grp.bf = shards[idx[0]].bf;
     grp.ntr = ntr;
     grp.nshards = n;
     long U = 0;

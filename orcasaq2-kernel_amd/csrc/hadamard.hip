@@ -25,7 +25,7 @@ __device__ __forceinline__ void had_zero(uint32_t* zero, int nzero)
 
 __global__ __launch_bounds__(64 * HAD_WAVES) void had_r_128_kernel(
     const uint4* in, uint4* out, const uint4* __restrict__ pre,  // in == out allowed
-    const uint4* __restrict__ post, float scale, long blocks, int blocks_per_row, uint32_t* zero, int nzero)
+    const uint4* __restrict__ post, float scale, long blocks, int blocks_per_row, uint32_t* zero, int nzero, int in_bf, int out_bf, long ld_out)
 {
     had_zero(zero, nzero);
     const long blk = ((long)blockIdx.x * HAD_WAVES + (threadIdx.x >> 6)) * 4 + ((threadIdx.x >> 4) & 3);
@@ -33,7 +33,8 @@ __global__ __launch_bounds__(64 * HAD_WAVES) void had_r_128_kernel(
     const int lane = threadIdx.x & 15;
     const int col_blk = (int)(blk % blocks_per_row);
     float v[8];
-    had_unpack(in[blk * 16 + lane], v);
+    const uint4 x = in[blk * 16 + lane];
+    had_unpack(uint4{act_pair(x.x, in_bf), act_pair(x.y, in_bf), act_pair(x.z, in_bf), act_pair(x.w, in_bf)}, v);
     if (pre) {
         float p[8];
         had_unpack(pre[col_blk * 16 + lane], p);
@@ -52,25 +53,21 @@ __global__ __launch_bounds__(64 * HAD_WAVES) void had_r_128_kernel(
     }
     uint32_t o[4];
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const uint16_t h0 = __builtin_bit_cast(uint16_t, (_Float16)(v[2 * i] * f[2 * i]));
-        const uint16_t h1 = __builtin_bit_cast(uint16_t, (_Float16)(v[2 * i + 1] * f[2 * i + 1]));
-        o[i] = (uint32_t)h0 | ((uint32_t)h1 << 16);
-    }
-    out[blk * 16 + lane] = uint4{o[0], o[1], o[2], o[3]};
+    for (int i = 0; i < 4; i++) o[i] = out_pair(v[2 * i] * f[2 * i], v[2 * i + 1] * f[2 * i + 1], out_bf);
+    out[(blk / blocks_per_row * ld_out + col_blk * 128) / 8 + lane] = uint4{o[0], o[1], o[2], o[3]};
 }
 
 // Pointers only 4-byte aligned: one wave per 128-block, lane l holds elements 2l, 2l + 1.
 __global__ __launch_bounds__(64 * HAD_WAVES) void had_r_128_narrow_kernel(
     const uint32_t* in, uint32_t* out, const uint32_t* __restrict__ pre,  // in == out allowed
-    const uint32_t* __restrict__ post, float scale, long blocks, int blocks_per_row, uint32_t* zero, int nzero)
+    const uint32_t* __restrict__ post, float scale, long blocks, int blocks_per_row, uint32_t* zero, int nzero, int in_bf, int out_bf, long ld_out)
 {
     had_zero(zero, nzero);
     const long blk = (long)blockIdx.x * HAD_WAVES + (threadIdx.x >> 6);
     if (blk >= blocks) return;  // no barriers in this kernel
     const int lane = threadIdx.x & 63;
     const int col_blk = (int)(blk % blocks_per_row);
-    const uint32_t v = in[blk * 64 + lane];
+    const uint32_t v = act_pair(in[blk * 64 + lane], in_bf);
     float v0 = (float)__builtin_bit_cast(_Float16, (uint16_t)(v & 0xffffu));
     float v1 = (float)__builtin_bit_cast(_Float16, (uint16_t)(v >> 16));
     if (pre) {
@@ -86,31 +83,31 @@ __global__ __launch_bounds__(64 * HAD_WAVES) void had_r_128_narrow_kernel(
     }
     v0 *= scale;
     v1 *= scale;
-    const uint16_t h0 = __builtin_bit_cast(uint16_t, (_Float16)v0);
-    const uint16_t h1 = __builtin_bit_cast(uint16_t, (_Float16)v1);
-    out[blk * 64 + lane] = (uint32_t)h0 | ((uint32_t)h1 << 16);
+    out[(blk / blocks_per_row * ld_out + col_blk * 128) / 2 + lane] = out_pair(v0, v1, out_bf);
 }
 
 int had_dispatch(const uint16_t* in, uint16_t* out, const uint16_t* pre, const uint16_t* post,
-                 float scale, long rows, int cols, hipStream_t stream, uint32_t* zero, int nzero)
+                 float scale, long rows, int cols, hipStream_t stream, uint32_t* zero, int nzero,
+                 int in_bf, int out_bf, long ld_out)
 {
+    if (ld_out == 0) ld_out = cols;
     const int bpr = cols / 128;
     const long blocks = rows * bpr;
     if (blocks == 0 && nzero == 0) return EXL3_OK;   // with words to clear: one workgroup, no blocks
     auto a16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
-    if (!a16(in) || !a16(out) || (pre && !a16(pre)) || (post && !a16(post))) {
+    if (!a16(in) || !a16(out) || ld_out % 8 || (pre && !a16(pre)) || (post && !a16(post))) {
         const long grid = std::max<long>(1, (blocks + HAD_WAVES - 1) / HAD_WAVES);
         hipLaunchKernelGGL(had_r_128_narrow_kernel, dim3((unsigned)grid), dim3(64 * HAD_WAVES), 0, stream,
                            reinterpret_cast<const uint32_t*>(in), reinterpret_cast<uint32_t*>(out),
                            reinterpret_cast<const uint32_t*>(pre), reinterpret_cast<const uint32_t*>(post),
-                           scale, blocks, bpr, zero, nzero);
+                           scale, blocks, bpr, zero, nzero, in_bf, out_bf, ld_out);
         return check_launch("exl3_had_r_128");
     }
     const long grid = std::max<long>(1, (blocks + 4 * HAD_WAVES - 1) / (4 * HAD_WAVES));
     hipLaunchKernelGGL(had_r_128_kernel, dim3((unsigned)grid), dim3(64 * HAD_WAVES), 0, stream,
                        reinterpret_cast<const uint4*>(in), reinterpret_cast<uint4*>(out),
                        reinterpret_cast<const uint4*>(pre), reinterpret_cast<const uint4*>(post),
-                       scale, blocks, bpr, zero, nzero);
+                       scale, blocks, bpr, zero, nzero, in_bf, out_bf, ld_out);
     return check_launch("exl3_had_r_128");
 }
 

@@ -1532,8 +1532,7 @@ int exl3r_gemm_sk(int mode, int rows, int ic, int nshards, const int* oc, const 
                          sk_ntiles(rows, oc[0]));
                 return emit(L);
             };
-            rc = sk_plan_single(fake_ptr<uint16_t>(B_AH), shards[0].trellis, shards[0].C, shards[0].svh, fake_ptr<char>(B_WS),
-                                ws, rows, ic, oc[0], K[0], cb[0], cus, emit_single);
+            rc = sk_plan_single(fake_ptr<uint16_t>(B_AH), shards[0], fake_ptr<char>(B_WS), ws, rows, cus, emit_single);
         } else {
             const char* what = "exl3_gemm_grouped";
             switch (bm) {

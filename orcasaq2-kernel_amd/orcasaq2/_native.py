@@ -16,13 +16,14 @@ import torch
 
 LIB_NAME = "libexl3hip.so"
 LIB_PATH = os.environ.get("ORCASAQ2_LIB", os.path.join(os.path.dirname(os.path.abspath(__file__)), LIB_NAME))
-ABI_VERSION = 7
+ABI_VERSION = 8
 
 CB_3INST, CB_MCG, CB_MUL1 = 0, 1, 2
 GEMV_MAX_ROWS = 16
 MAX_SHARDS = 64
 TOPK_MAX_K = 64
 TOPK_MAX_N = 1 << 19
+IO_DTYPES = {torch.float16: 0, torch.bfloat16: 1}
 
 _lib = None
 _lock = threading.Lock()
@@ -45,6 +46,9 @@ _SIGS = {
                                           ctypes.c_int, ctypes.c_int, ctypes.c_void_p]),
     "exl3_had_r_128": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p,
                                       ctypes.c_float, ctypes.c_long, ctypes.c_int, ctypes.c_void_p]),
+    "exl3_had_r_128_io": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p, ctypes.c_int, ctypes.c_long,
+                                         ctypes.c_void_p, ctypes.c_void_p, ctypes.c_float, ctypes.c_long,
+                                         ctypes.c_int, ctypes.c_void_p]),
     "exl3_gemv_workspace_bytes": (ctypes.c_size_t, [ctypes.c_int, ctypes.c_int, ctypes.c_int]),
     "exl3_gemv": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p,
                                  ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_int,
@@ -54,6 +58,9 @@ _SIGS = {
     "exl3_gemv_grouped": (ctypes.c_int, [ctypes.c_void_p, ctypes.POINTER(Shard), ctypes.c_int,
                                          ctypes.c_void_p, ctypes.c_size_t, ctypes.c_int, ctypes.c_int,
                                          ctypes.c_void_p]),
+    "exl3_gemv_grouped_io": (ctypes.c_int, [ctypes.c_void_p, ctypes.POINTER(Shard), ctypes.c_int, ctypes.c_int,
+                                            ctypes.c_void_p, ctypes.c_size_t, ctypes.c_int, ctypes.c_int,
+                                            ctypes.c_void_p]),
     "exl3_gemv_grouped_static": (ctypes.c_int, [ctypes.c_void_p, ctypes.POINTER(Shard), ctypes.c_int,
                                                 ctypes.c_int, ctypes.c_int, ctypes.c_void_p]),
     "exl3_gemm_workspace_bytes": (ctypes.c_size_t, [ctypes.c_int, ctypes.c_int, ctypes.c_int]),
@@ -65,6 +72,9 @@ _SIGS = {
     "exl3_gemm_grouped": (ctypes.c_int, [ctypes.c_void_p, ctypes.POINTER(Shard), ctypes.c_int,
                                          ctypes.c_void_p, ctypes.c_size_t, ctypes.c_int, ctypes.c_int,
                                          ctypes.c_void_p]),
+    "exl3_gemm_grouped_io": (ctypes.c_int, [ctypes.c_void_p, ctypes.POINTER(Shard), ctypes.c_int, ctypes.c_int,
+                                            ctypes.c_void_p, ctypes.c_size_t, ctypes.c_int, ctypes.c_int,
+                                            ctypes.c_void_p]),
     "exl3_embed_int8_gather": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int,
                                               ctypes.c_void_p, ctypes.c_void_p, ctypes.c_long,
                                               ctypes.c_int, ctypes.c_int, ctypes.c_void_p]),
@@ -283,6 +293,19 @@ def had_r_128(x: torch.Tensor, out: torch.Tensor | None = None, pre: torch.Tenso
     return out
 
 
+def had_r_128_cols(fn: str, x: torch.Tensor, out: torch.Tensor, col: int, pre: torch.Tensor | None = None,
+                   post: torch.Tensor | None = None) -> None:
+    """had_r_128 of x (rows, cols) fp16 or bf16 into columns col .. of the contiguous fp16 or bf16
+    `out` (rows, any): the typed loads and stores stand for the conversions around an fp16 call."""
+    rows, cols = x.shape
+    for name, v in (("pre", pre), ("post", post)):
+        if v is not None:
+            _vec16(fn, name, v, cols)
+    _need(out.is_contiguous() and out.shape[0] == rows and col + cols <= out.shape[1], fn, "out does not hold x")
+    _check(lib().exl3_had_r_128_io(_ptr(x), IO_DTYPES[x.dtype], out.data_ptr() + 2 * col, IO_DTYPES[out.dtype],
+                                   out.shape[1], _ptr(pre), _ptr(post), 1.0, rows, cols, _stream(x.device)), fn)
+
+
 def _shard_table(fn: str, x: torch.Tensor, shards: list[dict], out: torch.Tensor | None, dev):
     """(out, exl3_shard_t array) of a grouped call: the shards' outputs side by side in out
     (rows, sum oc), shard s writing its columns with row stride sum oc."""
@@ -290,8 +313,8 @@ def _shard_table(fn: str, x: torch.Tensor, shards: list[dict], out: torch.Tensor
     _need(1 <= len(shards) <= MAX_SHARDS, fn, f"{len(shards)} shards")
     total = sum(int(s["oc"]) for s in shards)
     if out is None:
-        out = torch.empty((rows, total), dtype=torch.float16, device=dev)
-    _need(out.dtype == torch.float16 and out.is_contiguous() and tuple(out.shape) == (rows, total), fn,
+        out = torch.empty((rows, total), dtype=x.dtype, device=dev)
+    _need(out.dtype == x.dtype and out.is_contiguous() and tuple(out.shape) == (rows, total), fn,
           f"out must be contiguous fp16 ({rows}, {total})")
     arr = (Shard * len(shards))()
     col = 0
@@ -322,6 +345,29 @@ def gemv_grouped(x: torch.Tensor, shards: list[dict], out: torch.Tensor | None =
     nbytes = L.exl3_gemv_grouped_workspace_bytes(arr, len(shards), rows, ic)
     ws = gemv_workspace(dev, nbytes)
     _check(L.exl3_gemv_grouped(_ptr(x), arr, len(shards), _ptr(ws), ws.numel(), rows, ic, _stream(dev)), fn)
+    return out
+
+
+def grouped_io(x: torch.Tensor, shards: list[dict]) -> torch.Tensor:
+    """gemv_grouped (up to GEMV_MAX_ROWS rows) or gemm_grouped of fp16 or bf16 x (rows, ic), the
+    outputs in x's dtype: bf16 activations are rounded to fp16 and fp16 outputs to bf16 in the
+    kernels' loads and stores."""
+    rows, ic = x.shape
+    gemv = rows <= GEMV_MAX_ROWS
+    fn = "exl3_gemv" if gemv else "exl3_gemm_grouped"
+    _need(x.dtype in IO_DTYPES and x.is_contiguous(), fn, "x must be contiguous fp16 or bf16")
+    dev = _need_gpu(fn, x, *[s["trellis"] for s in shards])
+    out, arr = _shard_table(fn, x, shards, None, dev)
+    L = lib()
+    io, n = IO_DTYPES[x.dtype], len(shards)
+    if gemv:
+        ws = gemv_workspace(dev, L.exl3_gemv_grouped_workspace_bytes(arr, n, rows, ic))
+        rc = L.exl3_gemv_grouped_io(_ptr(x), arr, n, io, _ptr(ws), ws.numel(), rows, ic, _stream(dev))
+    else:
+        nbytes = L.exl3_gemm_grouped_workspace_bytes(arr, n, rows, ic)
+        ws = workspace(dev, nbytes)
+        rc = L.exl3_gemm_grouped_io(_ptr(x), arr, n, io, _ptr(ws), nbytes, rows, ic, _stream(dev))
+    _check(rc, fn)
     return out
 
 

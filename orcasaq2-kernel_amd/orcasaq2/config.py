@@ -312,8 +312,26 @@ class Exl3LinearMethod(LinearMethodBase):
         if layer.exl3_shards is None:
             out = torch.nn.functional.linear(x, layer.exl3_dense.to(x.dtype))
             return out + bias if bias is not None else out
-        out = self.apply_fp16(layer, x).to(x.dtype)
+        if x.is_cuda and x.dtype in (torch.half, torch.bfloat16):
+            out = self._apply_io(layer, x)
+        else:
+            out = self.apply_fp16(layer, x).to(x.dtype)
         return out + bias if bias is not None else out
+
+    def _apply_io(self, layer, x: torch.Tensor) -> torch.Tensor:
+        """apply's fp16 and bf16 calls on the GPU: one op for the layer's shards, outputs in
+        x.dtype."""
+        rows = x.numel() // x.shape[-1]
+        xf = x.reshape(rows, x.shape[-1])
+        if not xf.is_contiguous():
+            xf = xf.contiguous()
+        if xf.dtype == torch.bfloat16 and xf.data_ptr() % 4:
+            xf = xf.clone()   # the kernels load pairs; a converted copy was always aligned
+        shards = layer.exl3_shards
+        out = torch.ops.orcasaq2.shards_linear(
+            xf, [s.trellis for s in shards], [s.suh for s in shards], [s.svh for s in shards],
+            [s.oc for s in shards], [float(s.K) for s in shards], [s.mcg for s in shards], [s.mul1 for s in shards])
+        return out.reshape(*x.shape[:-1], out.shape[-1])
 
     def apply_fp16(self, layer, x: torch.Tensor) -> torch.Tensor:
         """The shards' fp16 outputs of apply, before the cast to x.dtype and the bias."""
@@ -324,7 +342,7 @@ class Exl3LinearMethod(LinearMethodBase):
         if not xf.is_contiguous():
             xf = xf.contiguous()
         shards = layer.exl3_shards
-        route = _ops._op_route if xf.is_cuda else _ops._fused_route
+        route = _ops._op_route if xf.is_cuda else _ops._fused_route   # (the GPU's fp32 callers)
         if len(shards) > 1 and 0 < rows and (rows <= _ops.GEMM_MAX_ROWS or all(
                 route(rows, xf.shape[-1], s.oc) for s in shards)):
             grouped = torch.ops.orcasaq2.shards_gemv if rows <= GEMV_MAX_ROWS else torch.ops.orcasaq2.shards_gemm

@@ -175,3 +175,43 @@ def shards_gemm(x: Tensor, trellis: list[Tensor], suh: list[Tensor], svh: list[T
 @shards_gemm.register_fake
 def _shards_gemm_fake(x, trellis, suh, svh, oc, k, mcg, mul1) -> Tensor:
     return x.new_empty((x.shape[0], sum(oc)), dtype=torch.half)
+
+
+@torch.library.custom_op("orcasaq2::shards_linear", mutates_args=(), device_types="cuda")
+def shards_linear(x: Tensor, trellis: list[Tensor], suh: list[Tensor], svh: list[Tensor],
+                  oc: list[int], k: list[float], mcg: list[bool], mul1: list[bool]) -> Tensor:
+    """A layer's shards for any row count, fp16 or bf16 x in and out: what
+    orcasaq2/config.py:228-245 does around the shard op -- x to fp16, the shards' outputs side by
+    side, back to x's dtype -- with the conversions and the concatenation in the kernels' loads and
+    stores.  Separate passes cost a bf16 decoder layer ~40 us at one row (eight launches) and
+    ~420 us at 2048 rows; the concatenation 206 us of a gate_up call at 4096 rows."""
+    rows, ic = x.shape
+    cb = [_native.codebook_id(m, m1) for m, m1 in zip(mcg, mul1)]
+    if rows == 0:
+        return x.new_empty((0, sum(oc)))
+    if rows <= GEMV_MAX_ROWS or all(_op_route(rows, ic, o) for o in oc):
+        return _native.grouped_io(x, [dict(trellis=t, suh=a, svh=b, oc=o, K=kk, codebook=c)
+                                      for t, a, b, o, kk, c in zip(trellis, suh, svh, oc, k, cb)])
+    fn = "orcasaq2::shards_linear"
+    out = x.new_empty((rows, sum(oc)))
+    col = 0
+    for t, a, b, o, kk, c in zip(trellis, suh, svh, oc, k, cb):
+        if _op_route(rows, ic, o):
+            y = _native.grouped_io(x, [dict(trellis=t, suh=a, svh=b, oc=o, K=kk, codebook=c)])
+            out[:, col:col + o].copy_(y)
+        else:
+            # the reconstruct branch (see _reconstruct_branch)
+            xh = torch.empty((rows, ic), dtype=torch.half, device=x.device)
+            _native.had_r_128_cols(fn, x, xh, 0, pre=a)
+            wt = _native.reconstruct_t(t, kk, c)
+            y = torch.nn.functional.linear(xh, wt)
+            del wt, xh
+            _native.had_r_128_cols(fn, y, out, col, post=b)
+        del y
+        col += o
+    return out
+
+
+@shards_linear.register_fake
+def _shards_linear_fake(x, trellis, suh, svh, oc, k, mcg, mul1) -> Tensor:
+    return x.new_empty((x.shape[0], sum(oc)))

@@ -1,0 +1,50 @@
+"""bfloat16 activations and outputs inside the kernels' loads and stores (the op
+orcasaq2::shards_linear behind Exl3LinearMethod.apply): bit for bit what converting x to fp16, the
+fp16 ops, and converting the concatenated outputs back give, on every route -- one to four rows,
+five to sixteen, the K-split GEMM, the stream-K GEMM (one shard and grouped) and the reconstruct
+branch into its columns -- with values that round to fp16 infinity and outputs that are NaN."""
+import pytest
+import torch
+
+from orcasaq2 import _native
+from orcasaq2 import ops as O
+from orcasaq2 import synthetic as syn
+
+pytestmark = pytest.mark.gpu
+D = torch.device("cuda", 0)
+
+
+def _bits(t):
+    return torch.where(t.isnan(), torch.full_like(t, 7.0), t).view(torch.int16)
+
+
+@pytest.mark.parametrize("rows,ic,spec", [
+    (1, 384, [(256, 4)]), (1, 17408, [(128, 3)]),       # a whole segment; split into accumulator words
+    (4, 640, [(256, 3), (128, 5)]),
+    (9, 384, [(256, 4), (128, 2)]),
+    (33, 640, [(256, 3), (128, 6)]), (129, 384, [(128, 4)]),
+    (600, 8192, [(128, 4)]), (2000, 4096, [(8192, 2), (8192, 3)]),   # stream-K: one shard, grouped
+    (600, 640, [(256, 4), (128, 5)]),                    # the reconstruct branch
+    (515, 8192, [(128, 4), (256, 3)]),
+])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_typed_io_is_conversion_around_fp16(native, rows, ic, spec, dtype):
+    print(f"typed io rows={rows} ic={ic} {spec} {dtype}", flush=True)
+    g = torch.Generator(device=D).manual_seed(rows)
+    lins = [syn.linear_gpu(ic, oc, K, g, D) for oc, K in spec]
+    x = (torch.randn(rows, ic, generator=g, device=D) * 3).to(dtype)
+    if dtype == torch.bfloat16:
+        x[rows // 2, 5] = 1e6            # infinity in fp16
+    a = ([l["trellis"] for l in lins], [l["suh"] for l in lins], [l["svh"] for l in lins], [oc for oc, _ in spec],
+         [float(K) for _, K in spec], [False] * len(spec), [False] * len(spec))
+    got = torch.ops.orcasaq2.shards_linear(x, *a)
+    assert got.dtype == dtype and got.shape == (rows, sum(oc for oc, _ in spec))
+    xh = x.half()
+    shards = [dict(l, codebook=0) for l in lins]
+    if rows <= 16:
+        want = _native.gemv_grouped(xh, shards)
+    elif all(O._op_route(rows, ic, oc) for oc, _ in spec):
+        want = _native.gemm_grouped(xh, shards)
+    else:
+        want = torch.cat([O._shard_gemm_impl(xh, *(v[i] for v in a)) for i in range(len(spec))], dim=1)
+    assert torch.equal(_bits(got), _bits(want.to(dtype)))
