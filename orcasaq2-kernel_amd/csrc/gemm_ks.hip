@@ -27,6 +27,8 @@
 #include "exl3_common.h"
 #include "gemm_ks_plan.h"
 
+#include <atomic>
+
 namespace exl3 {
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
@@ -479,6 +481,19 @@ static const void* ks_fn(int mt)
     }
 }
 
+// The kernel's opt-in to its LDS (above 64 KiB), once per device and kernel: ~1 us of host time.
+static void ks_lds_optin(const void* fn, int mt, int cb)
+{
+    static std::atomic<uint32_t> done[64];
+    int dev = 0;
+    (void)hipGetDevice(&dev);
+    const uint32_t bit = 1u << (4 * cb + mt - 1);
+    if (dev < 64 && (done[dev].load(std::memory_order_relaxed) & bit)) return;
+    const hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, ks_lds(mt));
+    (void)hipGetLastError();
+    if (e == hipSuccess && dev < 64) done[dev].fetch_or(bit, std::memory_order_relaxed);
+}
+
 size_t gemm_ks_shard_bytes(int rows, int ic, int oc) { return ks_shard_bytes(rows, ic, oc, device_cus()); }
 
 int gemm_ks_dispatch(const uint16_t* A, const GemvShard* shards, int nshards, int rows, char* ws, size_t ws_bytes,
@@ -490,8 +505,7 @@ int gemm_ks_dispatch(const uint16_t* A, const GemvShard* shards, int nshards, in
         int rc = check_launch(what);
         if (rc != EXL3_OK) return rc;
         const void* fn = L.cb == CB_MCG ? ks_fn<CB_MCG>(L.mt) : ks_fn<CB_3INST>(L.mt);
-        (void)hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, ks_lds(L.mt));
-        (void)hipGetLastError();
+        ks_lds_optin(fn, L.mt, L.cb);
         KsArgs a = *L.args;
         void* kargs[] = {&a};
         (void)hipLaunchKernel(fn, dim3((unsigned)L.G), dim3(128 * KS_NP), kargs, ks_lds(L.mt), stream);

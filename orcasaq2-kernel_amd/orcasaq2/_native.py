@@ -90,6 +90,8 @@ EXPORTED = tuple(_SIGS)
 def lib() -> ctypes.CDLL:
     """Loads libexl3hip.so (after torch, so the HIP runtime torch mapped is reused)."""
     global _lib
+    if _lib is not None:
+        return _lib
     with _lock:
         if _lib is None:
             if not os.path.exists(LIB_PATH):
@@ -348,27 +350,47 @@ def gemv_grouped(x: torch.Tensor, shards: list[dict], out: torch.Tensor | None =
     return out
 
 
-def grouped_io(x: torch.Tensor, shards: list[dict]) -> torch.Tensor:
-    """gemv_grouped (up to GEMV_MAX_ROWS rows) or gemm_grouped of fp16 or bf16 x (rows, ic), the
-    outputs in x's dtype: bf16 activations are rounded to fp16 and fp16 outputs to bf16 in the
-    kernels' loads and stores."""
+def linear_io(x: torch.Tensor, out: torch.Tensor, col: int, trellis, suh, svh, oc, k, codebook) -> None:
+    """Shards that share x (rows, ic), fp16 or bf16, as gemv_grouped (up to GEMV_MAX_ROWS rows) or
+    gemm_grouped runs them, into columns col .. of the contiguous `out` (rows, any) of x's dtype:
+    bf16 activations are rounded to fp16 and fp16 outputs to bf16 in the kernels' loads and stores.
+    Lists of one entry per shard.  (One pass over the shards with the checks written out: an eager
+    call at few rows costs the host more than the GPU.)"""
     rows, ic = x.shape
     gemv = rows <= GEMV_MAX_ROWS
     fn = "exl3_gemv" if gemv else "exl3_gemm_grouped"
-    _need(x.dtype in IO_DTYPES and x.is_contiguous(), fn, "x must be contiguous fp16 or bf16")
-    dev = _need_gpu(fn, x, *[s["trellis"] for s in shards])
-    out, arr = _shard_table(fn, x, shards, None, dev)
+    io = IO_DTYPES.get(x.dtype)
+    _need(io is not None and x.is_contiguous(), fn, "x must be contiguous fp16 or bf16")
+    dev = x.device
+    n = len(trellis)
+    _need(1 <= n <= MAX_SHARDS, fn, f"{n} shards")
+    arr = (Shard * n)()
+    ld = out.shape[1]
+    base = out.data_ptr()
+    half = torch.float16
+    for i, t in enumerate(trellis):
+        a, b, o = suh[i], svh[i], oc[i]
+        if t.device != dev:
+            _need_gpu(fn, x, t)
+        K = check_trellis(fn, t, ic, o, k[i])
+        if not (a.dtype == half and b.dtype == half and a.numel() == ic and b.numel() == o and a.is_contiguous()
+                and b.is_contiguous()):
+            _vec16(fn, "suh", a, ic)
+            _vec16(fn, "svh", b, o)
+        arr[i] = Shard(t.data_ptr(), a.data_ptr(), b.data_ptr(), base + 2 * col, ld, o, K, codebook[i])
+        col += o
+    _need(col <= ld and out.shape[0] == rows and out.dtype == x.dtype and out.is_contiguous(), fn, "out does not hold the shards")
     L = lib()
-    io, n = IO_DTYPES[x.dtype], len(shards)
+    stream = torch.cuda.current_stream(dev).cuda_stream
     if gemv:
         ws = gemv_workspace(dev, L.exl3_gemv_grouped_workspace_bytes(arr, n, rows, ic))
-        rc = L.exl3_gemv_grouped_io(_ptr(x), arr, n, io, _ptr(ws), ws.numel(), rows, ic, _stream(dev))
+        rc = L.exl3_gemv_grouped_io(x.data_ptr(), arr, n, io, ws.data_ptr(), ws.numel(), rows, ic, stream)
     else:
         nbytes = L.exl3_gemm_grouped_workspace_bytes(arr, n, rows, ic)
         ws = workspace(dev, nbytes)
-        rc = L.exl3_gemm_grouped_io(_ptr(x), arr, n, io, _ptr(ws), nbytes, rows, ic, _stream(dev))
-    _check(rc, fn)
-    return out
+        rc = L.exl3_gemm_grouped_io(x.data_ptr(), arr, n, io, ws.data_ptr(), nbytes, rows, ic, stream)
+    if rc:
+        _check(rc, fn)
 
 
 def gemv(x, trellis, suh, svh, K, codebook, out=None) -> torch.Tensor:

@@ -321,17 +321,14 @@ class Exl3LinearMethod(LinearMethodBase):
     def _apply_io(self, layer, x: torch.Tensor) -> torch.Tensor:
         """apply's fp16 and bf16 calls on the GPU: one op for the layer's shards, outputs in
         x.dtype."""
-        rows = x.numel() // x.shape[-1]
-        xf = x.reshape(rows, x.shape[-1])
+        xf = x if x.dim() == 2 else x.reshape(x.numel() // x.shape[-1], x.shape[-1])
         if not xf.is_contiguous():
             xf = xf.contiguous()
-        if xf.dtype == torch.bfloat16 and xf.data_ptr() % 4:
-            xf = xf.clone()   # the kernels load pairs; a converted copy was always aligned
         shards = layer.exl3_shards
-        out = torch.ops.orcasaq2.shards_linear(
+        out = _ops.shards_linear_op(xf)(
             xf, [s.trellis for s in shards], [s.suh for s in shards], [s.svh for s in shards],
             [s.oc for s in shards], [float(s.K) for s in shards], [s.mcg for s in shards], [s.mul1 for s in shards])
-        return out.reshape(*x.shape[:-1], out.shape[-1])
+        return out if x.dim() == 2 else out.reshape(*x.shape[:-1], out.shape[-1])
 
     def apply_fp16(self, layer, x: torch.Tensor) -> torch.Tensor:
         """The shards' fp16 outputs of apply, before the cast to x.dtype and the bias."""

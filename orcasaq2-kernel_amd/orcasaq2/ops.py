@@ -177,28 +177,23 @@ def _shards_gemm_fake(x, trellis, suh, svh, oc, k, mcg, mul1) -> Tensor:
     return x.new_empty((x.shape[0], sum(oc)), dtype=torch.half)
 
 
-@torch.library.custom_op("orcasaq2::shards_linear", mutates_args=(), device_types="cuda")
-def shards_linear(x: Tensor, trellis: list[Tensor], suh: list[Tensor], svh: list[Tensor],
-                  oc: list[int], k: list[float], mcg: list[bool], mul1: list[bool]) -> Tensor:
-    """A layer's shards for any row count, fp16 or bf16 x in and out: what
-    orcasaq2/config.py:228-245 does around the shard op -- x to fp16, the shards' outputs side by
-    side, back to x's dtype -- with the conversions and the concatenation in the kernels' loads and
-    stores.  Separate passes cost a bf16 decoder layer ~40 us at one row (eight launches) and
-    ~420 us at 2048 rows; the concatenation 206 us of a gate_up call at 4096 rows."""
+def _shards_linear_impl(x: Tensor, trellis: list[Tensor], suh: list[Tensor], svh: list[Tensor],
+                        oc: list[int], k: list[float], mcg: list[bool], mul1: list[bool]) -> Tensor:
     rows, ic = x.shape
     cb = [_native.codebook_id(m, m1) for m, m1 in zip(mcg, mul1)]
-    if rows == 0:
-        return x.new_empty((0, sum(oc)))
-    if rows <= GEMV_MAX_ROWS or all(_op_route(rows, ic, o) for o in oc):
-        return _native.grouped_io(x, [dict(trellis=t, suh=a, svh=b, oc=o, K=kk, codebook=c)
-                                      for t, a, b, o, kk, c in zip(trellis, suh, svh, oc, k, cb)])
-    fn = "orcasaq2::shards_linear"
     out = x.new_empty((rows, sum(oc)))
+    if rows == 0:
+        return out
+    if x.dtype == torch.bfloat16 and x.data_ptr() % 4:
+        x = x.clone()   # the kernels load pairs; a copy converted to fp16 was always aligned
+    if rows <= GEMV_MAX_ROWS or all(_op_route(rows, ic, o) for o in oc):
+        _native.linear_io(x, out, 0, trellis, suh, svh, oc, k, cb)
+        return out
+    fn = "orcasaq2::shards_linear"
     col = 0
     for t, a, b, o, kk, c in zip(trellis, suh, svh, oc, k, cb):
         if _op_route(rows, ic, o):
-            y = _native.grouped_io(x, [dict(trellis=t, suh=a, svh=b, oc=o, K=kk, codebook=c)])
-            out[:, col:col + o].copy_(y)
+            _native.linear_io(x, out, col, [t], [a], [b], [o], [kk], [c])
         else:
             # the reconstruct branch (see _reconstruct_branch)
             xh = torch.empty((rows, ic), dtype=torch.half, device=x.device)
@@ -207,11 +202,41 @@ def shards_linear(x: Tensor, trellis: list[Tensor], suh: list[Tensor], svh: list
             y = torch.nn.functional.linear(xh, wt)
             del wt, xh
             _native.had_r_128_cols(fn, y, out, col, post=b)
-        del y
+            del y
         col += o
     return out
+
+
+@torch.library.custom_op("orcasaq2::shards_linear", mutates_args=(), device_types="cuda")
+def shards_linear(x: Tensor, trellis: list[Tensor], suh: list[Tensor], svh: list[Tensor],
+                  oc: list[int], k: list[float], mcg: list[bool], mul1: list[bool]) -> Tensor:
+    """A layer's shards for any row count, fp16 or bf16 x in and out: what
+    orcasaq2/config.py:228-245 does around the shard op -- x to fp16, the shards' outputs side by
+    side, back to x's dtype -- with the conversions and the concatenation in the kernels' loads and
+    stores.  Separate passes cost a bf16 decoder layer ~40 us at one row (eight launches) and
+    ~420 us at 2048 rows; the concatenation 206 us of a gate_up call at 4096 rows."""
+    return _shards_linear_impl(x, trellis, suh, svh, oc, k, mcg, mul1)
 
 
 @shards_linear.register_fake
 def _shards_linear_fake(x, trellis, suh, svh, oc, k, mcg, mul1) -> Tensor:
     return x.new_empty((x.shape[0], sum(oc)))
+
+
+# The same op without custom_op's Python wrapper, for eager calls that need no gradient: the wrapper
+# (an autograd kernel that refuses backward, checks of the outputs) costs ~15 us of host time per
+# call (23-25 us against 8-10 with three shards), as long as a decode launch runs.
+_eager = torch.library.Library("orcasaq2", "FRAGMENT")
+_eager.define("shards_linear_eager(Tensor x, Tensor[] trellis, Tensor[] suh, Tensor[] svh, int[] oc, float[] k, "
+              "bool[] mcg, bool[] mul1) -> Tensor")
+_eager.impl("shards_linear_eager", _shards_linear_impl, "CUDA")
+torch.library.register_fake("orcasaq2::shards_linear_eager", _shards_linear_fake, lib=_eager)
+
+
+def shards_linear_op(x: Tensor):
+    """shards_linear, or its eager form where nothing could ask for a derivative of the call:
+    not being compiled, no gradient wanted of x, no forward-mode level open."""
+    if (torch.compiler.is_compiling() or (x.requires_grad and torch.is_grad_enabled())
+            or torch.autograd.forward_ad._current_level >= 0):
+        return torch.ops.orcasaq2.shards_linear
+    return torch.ops.orcasaq2.shards_linear_eager

@@ -39,6 +39,7 @@ def test_typed_io_is_conversion_around_fp16(native, rows, ic, spec, dtype):
          [float(K) for _, K in spec], [False] * len(spec), [False] * len(spec))
     got = torch.ops.orcasaq2.shards_linear(x, *a)
     assert got.dtype == dtype and got.shape == (rows, sum(oc for oc, _ in spec))
+    assert torch.equal(_bits(torch.ops.orcasaq2.shards_linear_eager(x, *a)), _bits(got))
     xh = x.half()
     shards = [dict(l, codebook=0) for l in lins]
     if rows <= 16:
@@ -48,3 +49,25 @@ def test_typed_io_is_conversion_around_fp16(native, rows, ic, spec, dtype):
     else:
         want = torch.cat([O._shard_gemm_impl(xh, *(v[i] for v in a)) for i in range(len(spec))], dim=1)
     assert torch.equal(_bits(got), _bits(want.to(dtype)))
+
+
+def test_gradient_of_the_layer_is_still_refused(native):
+    """An x that requires a gradient takes the op whose backward raises, not the eager form."""
+    from orcasaq2.config import Exl3Config, Exl3LinearMethod
+    layer, method = torch.nn.Module(), Exl3LinearMethod(Exl3Config.from_config({}), "p")
+    method.create_weights(layer, 256, [128], 256, 128, torch.half)
+    lin = syn.linear(256, 128, 4, seed=1)
+    for name in ("trellis", "suh", "svh"):
+        getattr(layer, name).weight_loader(getattr(layer, name), lin[name].to(D))
+    method.process_weights_after_loading(layer)
+    x = torch.randn(2, 256, device=D).half()
+    y = method.apply(layer, x.clone().requires_grad_())
+    with pytest.raises(RuntimeError):
+        y.float().sum().backward()
+    assert torch.equal(method.apply(layer, x), y.detach())
+    for v in (x, x.bfloat16()):
+        got = torch.compile(lambda t: method.apply(layer, t * 1.0), backend="eager", fullgraph=True)(v)
+        assert torch.equal(got, method.apply(layer, v))
+    # bf16 at an odd element offset: as good as an aligned copy
+    flat = torch.cat([x.flatten()[:1], x.flatten()]).bfloat16()
+    assert torch.equal(method.apply(layer, flat[1:].view(2, 256)), method.apply(layer, x.bfloat16()))
