@@ -194,9 +194,15 @@ size_t exl3_gemm_grouped_workspace_bytes(const exl3_shard_t* shards, int nshards
 int exl3_gemm_grouped(const void* A, const exl3_shard_t* shards, int nshards, void* workspace,
                       size_t ws_bytes, int rows, int ic, void* stream);
 
-/* exl3_gemm_grouped with A and every C of type io_dtype (see exl3_gemv_grouped_io). */
-int exl3_gemm_grouped_io(const void* A, const exl3_shard_t* shards, int nshards, int io_dtype, void* workspace,
-                         size_t ws_bytes, int rows, int ic, void* stream);
+/*
+ * exl3_gemm_grouped with A and every C of type io_dtype (see exl3_gemv_grouped_io).  ksplit 0: the
+ * kernel by row count, as exl3_gemm_grouped; else the K-split decode-GEMM at any row count (for
+ * layers whose library GEMMs are too small to beat it), with a workspace of
+ * exl3_gemm_ksplit_workspace_bytes.
+ */
+size_t exl3_gemm_ksplit_workspace_bytes(const exl3_shard_t* shards, int nshards, int rows, int ic);
+int exl3_gemm_grouped_io(const void* A, const exl3_shard_t* shards, int nshards, int io_dtype, int ksplit,
+                         void* workspace, size_t ws_bytes, int rows, int ic, void* stream);
 
 /*
  * int8 embedding gather: out[n, :] = dtype(table[ids[n], :]) * scales[ids[n]], computed

@@ -241,14 +241,25 @@ size_t exl3_gemm_grouped_workspace_bytes(const exl3_shard_t* shards, int nshards
     return t;
 }
 
+size_t exl3_gemm_ksplit_workspace_bytes(const exl3_shard_t* shards, int nshards, int rows, int ic)
+{
+    if (!shards || nshards < 1 || rows < 1 || ic < 128) return 0;
+    size_t t = 0;
+    for (int i = 0; i < nshards; i++) {
+        if (shards[i].oc < 128) return 0;
+        t += gemm_ks_shard_bytes(rows, ic, shards[i].oc);
+    }
+    return t;
+}
+
 int exl3_gemm_grouped(const void* A, const exl3_shard_t* shards, int nshards, void* workspace, size_t ws_bytes,
                       int rows, int ic, void* stream)
 {
-    return exl3_gemm_grouped_io(A, shards, nshards, EXL3_IO_F16, workspace, ws_bytes, rows, ic, stream);
+    return exl3_gemm_grouped_io(A, shards, nshards, EXL3_IO_F16, 0, workspace, ws_bytes, rows, ic, stream);
 }
 
-int exl3_gemm_grouped_io(const void* A, const exl3_shard_t* shards, int nshards, int io_dtype, void* workspace,
-                         size_t ws_bytes, int rows, int ic, void* stream)
+int exl3_gemm_grouped_io(const void* A, const exl3_shard_t* shards, int nshards, int io_dtype, int ksplit,
+                         void* workspace, size_t ws_bytes, int rows, int ic, void* stream)
 {
     g_err[0] = 0;
     const int bf = io_dtype;
@@ -260,7 +271,8 @@ int exl3_gemm_grouped_io(const void* A, const exl3_shard_t* shards, int nshards,
     if (rows < 1) return set_error(EXL3_ERR_ARG, "exl3_gemm_grouped: rows=%d", rows);
     if (!aligned(A, 4) || !aligned(workspace, 256))
         return set_error(EXL3_ERR_ARG, "exl3_gemm_grouped: A must be 4-byte and workspace 256-byte aligned");
-    const size_t need = exl3_gemm_grouped_workspace_bytes(shards, nshards, rows, ic);
+    const size_t need = ksplit ? exl3_gemm_ksplit_workspace_bytes(shards, nshards, rows, ic)
+                               : exl3_gemm_grouped_workspace_bytes(shards, nshards, rows, ic);
     GemvShard d[EXL3_MAX_SHARDS];
     for (int i = 0; i < nshards; i++) {
         const exl3_shard_t& s = shards[i];
@@ -275,6 +287,9 @@ int exl3_gemm_grouped_io(const void* A, const exl3_shard_t* shards, int nshards,
     }
     if (ws_bytes < need)
         return set_error(EXL3_ERR_WORKSPACE, "exl3_gemm_grouped: workspace of %zu bytes, %zu needed", ws_bytes, need);
+    if (ksplit)
+        return gemm_ks_dispatch(static_cast<const uint16_t*>(A), d, nshards, rows, static_cast<char*>(workspace), ws_bytes,
+                                static_cast<hipStream_t>(stream), "exl3_gemm_grouped");
     return gemm_grouped_dispatch(static_cast<const uint16_t*>(A), d, nshards, rows, static_cast<char*>(workspace),
                                  ws_bytes, static_cast<hipStream_t>(stream));
 }

@@ -19,8 +19,10 @@ constexpr int KS_MAXSH = 8;        // shards per launch
 constexpr int KS_PIN = 32;         // inputs per step (two tile rows)
 constexpr int KS_LDQ = 36;         // floats per staged column of 32 rows (padded)
 constexpr int KS_LDC = 132;        // floats per row of the output staging
-constexpr int KS_MIN_STEPS = 2;    // least steps per pair a launch is spread for (below, a pair's
-                                   // steps cost less than its slot)
+// Least steps per pair a launch is spread for: below, splitting further costs more in slots than
+// it saves in steps (2048 -> 2048 at 24 rows, 1 / 2 / 4 steps: 13.5 / 12.6 / 13.7 us per call;
+// 2048 -> 2048 + 2 x 512 at 128 rows, 2 / 4 / 8: 24.4 / 21.7 / 23.6).
+KS_HD constexpr int ks_min_steps(int mt) { return mt == 1 ? 2 : 4; }
 constexpr int KS_NP = 4;           // wave pairs of a workgroup: a pair shares its steps, 64 outputs each wave
 constexpr int KS_WBYTES = 2048;    // LDS of a wave's trellis words of one step (64 lanes x 8 words)
 
@@ -201,10 +203,10 @@ inline size_t ks_ah_bytes(int rows, int ic)
     return ks_align((size_t)t.nrt * t.mt * 32 * ic * 2);
 }
 
-// Workgroups of a launch: one per CU, fewer where a pair would get under KS_MIN_STEPS steps.
-inline int ks_wgs(long steps, int cus)
+// Workgroups of a launch: one per CU, fewer where a pair would get under ks_min_steps steps.
+inline int ks_wgs(long steps, int mt, int cus)
 {
-    return (int)std::min<long>(cus, std::max<long>(1, steps / (KS_NP * KS_MIN_STEPS)));
+    return (int)std::min<long>(cus, std::max<long>(1, steps / (KS_NP * ks_min_steps(mt))));
 }
 
 // A shard's share of a call's workspace: its activations, and slots for its segments and the
@@ -266,7 +268,7 @@ int ks_plan(const uint16_t* A, const GemvShard* shards, int nshards, int rows, c
         }
         a.nrt = t.nrt;
         const int nsegs = t.nrt * ncg;
-        a.G = ks_wgs((long)nsegs * a.P, cus);
+        a.G = ks_wgs((long)nsegs * a.P, t.mt, cus);
         a.full = nsegs / a.G;
         a.nrem = nsegs % a.G;
         const int np = KS_NP * a.G;

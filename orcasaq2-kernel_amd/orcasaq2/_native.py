@@ -72,9 +72,11 @@ _SIGS = {
     "exl3_gemm_grouped": (ctypes.c_int, [ctypes.c_void_p, ctypes.POINTER(Shard), ctypes.c_int,
                                          ctypes.c_void_p, ctypes.c_size_t, ctypes.c_int, ctypes.c_int,
                                          ctypes.c_void_p]),
+    "exl3_gemm_ksplit_workspace_bytes": (ctypes.c_size_t, [ctypes.POINTER(Shard), ctypes.c_int, ctypes.c_int,
+                                                           ctypes.c_int]),
     "exl3_gemm_grouped_io": (ctypes.c_int, [ctypes.c_void_p, ctypes.POINTER(Shard), ctypes.c_int, ctypes.c_int,
-                                            ctypes.c_void_p, ctypes.c_size_t, ctypes.c_int, ctypes.c_int,
-                                            ctypes.c_void_p]),
+                                            ctypes.c_int, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_int,
+                                            ctypes.c_int, ctypes.c_void_p]),
     "exl3_embed_int8_gather": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int,
                                               ctypes.c_void_p, ctypes.c_void_p, ctypes.c_long,
                                               ctypes.c_int, ctypes.c_int, ctypes.c_void_p]),
@@ -350,9 +352,10 @@ def gemv_grouped(x: torch.Tensor, shards: list[dict], out: torch.Tensor | None =
     return out
 
 
-def linear_io(x: torch.Tensor, out: torch.Tensor, col: int, trellis, suh, svh, oc, k, codebook) -> None:
+def linear_io(x: torch.Tensor, out: torch.Tensor, cols, trellis, suh, svh, oc, k, codebook, ksplit: bool = False) -> None:
     """Shards that share x (rows, ic), fp16 or bf16, as gemv_grouped (up to GEMV_MAX_ROWS rows) or
-    gemm_grouped runs them, into columns col .. of the contiguous `out` (rows, any) of x's dtype:
+    gemm_grouped runs them (ksplit: the K-split decode-GEMM at any row count), shard i into columns
+    cols[i] .. of the contiguous `out` (rows, any) of x's dtype:
     bf16 activations are rounded to fp16 and fp16 outputs to bf16 in the kernels' loads and stores.
     Lists of one entry per shard.  (One pass over the shards with the checks written out: an eager
     call at few rows costs the host more than the GPU.)"""
@@ -377,18 +380,19 @@ def linear_io(x: torch.Tensor, out: torch.Tensor, col: int, trellis, suh, svh, o
                 and b.is_contiguous()):
             _vec16(fn, "suh", a, ic)
             _vec16(fn, "svh", b, o)
-        arr[i] = Shard(t.data_ptr(), a.data_ptr(), b.data_ptr(), base + 2 * col, ld, o, K, codebook[i])
-        col += o
-    _need(col <= ld and out.shape[0] == rows and out.dtype == x.dtype and out.is_contiguous(), fn, "out does not hold the shards")
+        _need(cols[i] + o <= ld, fn, "out does not hold the shards")
+        arr[i] = Shard(t.data_ptr(), a.data_ptr(), b.data_ptr(), base + 2 * cols[i], ld, o, K, codebook[i])
+    _need(out.shape[0] == rows and out.dtype == x.dtype and out.is_contiguous(), fn, "out does not hold the shards")
     L = lib()
     stream = torch.cuda.current_stream(dev).cuda_stream
     if gemv:
         ws = gemv_workspace(dev, L.exl3_gemv_grouped_workspace_bytes(arr, n, rows, ic))
         rc = L.exl3_gemv_grouped_io(x.data_ptr(), arr, n, io, ws.data_ptr(), ws.numel(), rows, ic, stream)
     else:
-        nbytes = L.exl3_gemm_grouped_workspace_bytes(arr, n, rows, ic)
+        size = L.exl3_gemm_ksplit_workspace_bytes if ksplit else L.exl3_gemm_grouped_workspace_bytes
+        nbytes = size(arr, n, rows, ic)
         ws = workspace(dev, nbytes)
-        rc = L.exl3_gemm_grouped_io(x.data_ptr(), arr, n, io, ws.data_ptr(), nbytes, rows, ic, stream)
+        rc = L.exl3_gemm_grouped_io(x.data_ptr(), arr, n, io, ksplit, ws.data_ptr(), nbytes, rows, ic, stream)
     if rc:
         _check(rc, fn)
 

@@ -30,6 +30,7 @@ Dispatch on the number of activation rows (reference: orcasaq2/ops.py:25, 46-59)
 The op is registered for the "cuda" device type (ROCm) only: there is no CPU path.
 """
 
+import functools
 import os
 
 import torch
@@ -177,6 +178,52 @@ def _shards_gemm_fake(x, trellis, suh, svh, oc, k, mcg, mul1) -> Tensor:
     return x.new_empty((x.shape[0], sum(oc)), dtype=torch.half)
 
 
+# Above SPLIT_MAX_ROWS a layer's shards take the K-split decode-GEMM together where it beats their
+# own routes, by estimates (us on MI355X) fitted to HIP-graph timings at 520..4096 rows of 2048-,
+# 5120-, 6144- and 17408-input layers.  Measured, own routes / K split: qkv 5120 -> 6144 + 2 x 1024 at
+# 520, 1024, 1536, 2048 rows 150 / 94, 181 / 135, 217 / 197, 257 / 262; its k and v alone at 2048, 3072,
+# 4096 rows 113 / 84, 136 / 133, 162 / 163; gate_up 5120 -> 2 x 17408 at 520, 640, 768 rows 278 / 295,
+# 326 / 305, 341 / 365; 2048 -> 2 x 6144 at 1024, 1536 rows 106 / 99, 126 / 149; 17408 -> 5120 (stream-K)
+# at 640, 768, 1024 rows 185 / 156, 190 / 187, 225 / 240.
+_CUS = 256
+_SPLIT_MARGIN = 1.05   # the library GEMM is far from monotone: take the K split where it is clear
+
+
+def _ksplit_us(rows: int, ic: int, ocs) -> float:
+    """Whole rounds of 128 x 128-output segments, one per CU (fill, epilogue, then a step of 32
+    inputs per pair of waves), and the segments left over split evenly, with a finishing launch."""
+    full, rem = divmod(-(-rows // 128) * (sum(ocs) // 128), _CUS)
+    steps = ic / 32
+    us = 4 + 1e-6 * rows * ic * len(ocs) + full * (10 + 1.1 * steps / 4)
+    return us + (20 + 1.1 * rem * steps / (4 * _CUS) if rem else 0)
+
+
+def _own_us(rows: int, ic: int, oc: int) -> float:
+    """The shard's own route: the stream-K kernel where _fused_route takes it (256-row tiles and a
+    tail of its own), else the reconstruct branch (four launches, W_q written and read, the library
+    GEMM, two Hadamard passes)."""
+    mweights = ic * oc * 1e-6
+    if _fused_route(rows, ic, oc):
+        return 60 + 0.472 * -(-rows // 256) * mweights
+    return 28 + 0.4 * mweights + 0.18 * rows / 128 * mweights + 1e-6 * rows * (ic + oc)
+
+
+@functools.lru_cache(maxsize=1024)
+def _ksplit_shards(rows: int, ic: int, ocs: tuple) -> tuple:
+    """Shards (indices) of a layer above SPLIT_MAX_ROWS that run as one K-split call: the narrowest
+    ones, as many as give the least estimated time with the wider ones on their own routes."""
+    if GEMM_MAX_ROWS_SET:
+        return ()
+    idx = sorted(range(len(ocs)), key=lambda i: ocs[i])
+    own = [_own_us(rows, ic, ocs[i]) for i in idx]
+    best, take = sum(own), 0
+    for n in range(1, len(idx) + 1):
+        us = _SPLIT_MARGIN * _ksplit_us(rows, ic, [ocs[i] for i in idx[:n]]) + sum(own[n:])
+        if us < best:
+            best, take = us, n
+    return tuple(sorted(idx[:take]))
+
+
 def _shards_linear_impl(x: Tensor, trellis: list[Tensor], suh: list[Tensor], svh: list[Tensor],
                         oc: list[int], k: list[float], mcg: list[bool], mul1: list[bool]) -> Tensor:
     rows, ic = x.shape
@@ -186,24 +233,39 @@ def _shards_linear_impl(x: Tensor, trellis: list[Tensor], suh: list[Tensor], svh
         return out
     if x.dtype == torch.bfloat16 and x.data_ptr() % 4:
         x = x.clone()   # the kernels load pairs; a copy converted to fp16 was always aligned
-    if rows <= GEMV_MAX_ROWS or all(_op_route(rows, ic, o) for o in oc):
-        _native.linear_io(x, out, 0, trellis, suh, svh, oc, k, cb)
+    cols = [0]
+    for o in oc:
+        cols.append(cols[-1] + o)
+
+    def fused(idx, ksplit=False):
+        def pick(v):
+            return v if len(idx) == len(oc) else [v[i] for i in idx]
+        _native.linear_io(x, out, pick(cols), pick(trellis), pick(suh), pick(svh), pick(oc), pick(k), pick(cb), ksplit)
+
+    every = range(len(oc))
+    if rows <= GEMV_MAX_ROWS or (rows <= SPLIT_MAX_ROWS and _op_route(rows, ic, 0)):
+        fused(every)
+        return out
+    split = _ksplit_shards(rows, ic, tuple(oc)) if rows > SPLIT_MAX_ROWS else ()
+    if split:
+        fused(split, True)
+    rest = [i for i in every if i not in split]
+    if rest and all(_op_route(rows, ic, oc[i]) for i in rest):
+        fused(rest)
         return out
     fn = "orcasaq2::shards_linear"
-    col = 0
-    for t, a, b, o, kk, c in zip(trellis, suh, svh, oc, k, cb):
-        if _op_route(rows, ic, o):
-            _native.linear_io(x, out, col, [t], [a], [b], [o], [kk], [c])
-        else:
-            # the reconstruct branch (see _reconstruct_branch)
-            xh = torch.empty((rows, ic), dtype=torch.half, device=x.device)
-            _native.had_r_128_cols(fn, x, xh, 0, pre=a)
-            wt = _native.reconstruct_t(t, kk, c)
-            y = torch.nn.functional.linear(xh, wt)
-            del wt, xh
-            _native.had_r_128_cols(fn, y, out, col, post=b)
-            del y
-        col += o
+    for i in rest:
+        if _op_route(rows, ic, oc[i]):
+            fused([i])
+            continue
+        # the reconstruct branch (see _reconstruct_branch)
+        xh = torch.empty((rows, ic), dtype=torch.half, device=x.device)
+        _native.had_r_128_cols(fn, x, xh, 0, pre=suh[i])
+        wt = _native.reconstruct_t(trellis[i], k[i], cb[i])
+        y = torch.nn.functional.linear(xh, wt)
+        del wt, xh
+        _native.had_r_128_cols(fn, y, out, cols[i], post=svh[i])
+        del y
     return out
 
 

@@ -24,7 +24,9 @@ def _bits(t):
     (9, 384, [(256, 4), (128, 2)]),
     (33, 640, [(256, 3), (128, 6)]), (129, 384, [(128, 4)]),
     (600, 8192, [(128, 4)]), (2000, 4096, [(8192, 2), (8192, 3)]),   # stream-K: one shard, grouped
-    (600, 640, [(256, 4), (128, 5)]),                    # the reconstruct branch
+    (600, 640, [(256, 4), (128, 5)]),                    # above 512 rows: the K split at 600,
+    (2500, 5120, [(6144, 4), (128, 5), (256, 3)]),       # the narrow shards beside a reconstruct branch,
+    (1100, 5120, [(5120, 2)]),                           # the reconstruct branch alone
     (515, 8192, [(128, 4), (256, 3)]),
 ])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
@@ -42,12 +44,19 @@ def test_typed_io_is_conversion_around_fp16(native, rows, ic, spec, dtype):
     assert torch.equal(_bits(torch.ops.orcasaq2.shards_linear_eager(x, *a)), _bits(got))
     xh = x.half()
     shards = [dict(l, codebook=0) for l in lins]
+    split = O._ksplit_shards(rows, ic, tuple(oc for oc, _ in spec)) if rows > O.SPLIT_MAX_ROWS else ()
     if rows <= 16:
         want = _native.gemv_grouped(xh, shards)
-    elif all(O._op_route(rows, ic, oc) for oc, _ in spec):
+    elif not split and all(O._op_route(rows, ic, oc) for oc, _ in spec):
         want = _native.gemm_grouped(xh, shards)
     else:
-        want = torch.cat([O._shard_gemm_impl(xh, *(v[i] for v in a)) for i in range(len(spec))], dim=1)
+        want = torch.empty(rows, sum(a[3]), dtype=torch.half, device=D)
+        cols = [sum(a[3][:i]) for i in range(len(spec))]
+        if split:
+            _native.linear_io(xh, want, [cols[i] for i in split], *([v[i] for i in split] for v in a[:5]), [0] * len(split),
+                              True)
+        for i in set(range(len(spec))) - set(split):
+            want[:, cols[i]:cols[i] + a[3][i]] = O._shard_gemm_impl(xh, *(v[i] for v in a))
     assert torch.equal(_bits(got), _bits(want.to(dtype)))
 
 

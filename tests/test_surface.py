@@ -322,3 +322,19 @@ def test_fused_gemm_routing_follows_the_measured_crossovers():
         assert not r(1536, 5120, 17408) and not r(3073, 5120, 17408) and not r(4096, 5120, 17408)
     assert not r(145, 5120, 17408) and not r(1024, 5120, 17408)
     assert not r(2048, 5120, 6144) and not r(145, 512, 256) and not r(2048, 2048, 8192)
+
+
+def test_layer_route_above_512_rows_follows_the_estimates():
+    """Which shards of a layer take the K-split kernel together above 512 rows, at measured points
+    well away from the crossovers, and the row knob's hard switch."""
+    from orcasaq2 import ops
+    f = ops._ksplit_shards
+    if ops.GEMM_MAX_ROWS_SET:
+        assert f(1024, 5120, (6144, 1024, 1024)) == ()
+        return
+    assert f(1024, 5120, (6144, 1024, 1024)) == (0, 1, 2)
+    assert f(2048, 5120, (6144, 1024, 1024)) == (1, 2)       # q to the library GEMM, k and v together
+    assert f(8192, 5120, (6144, 1024, 1024)) == () and f(2048, 6144, (5120,)) == ()
+    assert f(2048, 5120, (17408, 17408)) == () and f(1024, 5120, (17408, 17408)) == ()
+    assert f(640, 17408, (5120,)) == (0,) and f(1024, 17408, (5120,)) == () and f(2048, 17408, (5120,)) == ()
+    assert f(1024, 2048, (6144, 6144)) == (0, 1) and f(2048, 2048, (6144, 6144)) == ()
