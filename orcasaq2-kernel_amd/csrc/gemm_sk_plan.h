@@ -18,9 +18,9 @@ namespace exl3 {
 #define SK_HD __host__ __device__ __forceinline__
 
 constexpr int SK_WAVES = 8;
+constexpr int SK_BM = 256;
 constexpr int SK_BN = 256;
 constexpr int SK_KS = 64;                     // inputs per K-step (4 tile rows)
-constexpr int SK_LD = SK_KS + 8;              // halves per LDS row of the A and B tiles
 constexpr int SK_CLD = 128 + 4;               // floats per epilogue row in LDS (BM = 256)
 constexpr int SK_MAXSH = 8;                   // shards per launch
 constexpr int SK_WPE = 2;                     // waves per SIMD the register budget is set for (one workgroup per CU)
@@ -30,28 +30,8 @@ template <int BM>
 struct SkCfg;
 template <>
 struct SkCfg<256> { static constexpr int WM = 2, WN = 4, MB = 8, NB = 4; };
-template <>
-struct SkCfg<128> { static constexpr int WM = 1, WN = 8, MB = 8, NB = 2; };
-template <>
-struct SkCfg<64> { static constexpr int WM = 1, WN = 8, MB = 4, NB = 2; };
-template <>
-struct SkCfg<96> { static constexpr int WM = 1, WN = 8, MB = 6, NB = 2; };
-template <>
-struct SkCfg<48> { static constexpr int WM = 1, WN = 8, MB = 3, NB = 2; };
-template <>
-struct SkCfg<32> { static constexpr int WM = 1, WN = 8, MB = 2, NB = 2; };
-
 template <int BM>
 constexpr int sk_acc() { return SkCfg<BM>::MB * SkCfg<BM>::NB * 4; }   // fp32 accumulators per lane
-// LDS of a launch: the A and B tiles of one K-step, twice (the tiles of step s + 1 are written
-// while the MFMAs read those of step s), one workgroup per CU.  Measured on MI355X at 17..64
-// rows: the two-buffer pipeline with one workgroup per CU beats one buffer with two
-// workgroups per CU by 28% on 17408 -> 5120 and 6% on 5120 -> 17408.
-template <int BM>
-constexpr int sk_buf() { return (BM + SK_BN) * SK_LD; }                   // halves per A + B buffer
-template <int BM>
-constexpr int sk_lds() { return 2 * sk_buf<BM>() * 2; }      // bytes
-
 struct SkShard {
     const uint16_t* Ah;        // (rows, ic) fp16, fp16(H(A * suh)) of this shard
     const uint32_t* trellis;   // (ic/16, oc/16, 8K) u32
@@ -59,7 +39,7 @@ struct SkShard {
     uint16_t* C;               // (rows, ldc) fp16, columns [0, oc)
     long ldc;
     int oc, ntn, tbeg;         // outputs, 256-wide tile columns, first tile of the shard
-    int K;                     // bits per weight (read by the per-shard-K kernel)
+    int K;                     // bits per weight (of every shard of a launch)
 };
 
 struct SkArgs {
@@ -146,54 +126,12 @@ SK_HD SkPiece sk_piece(const SkArgs& a, long u, long u_end)
 
 // ---------------------------------------------------------------- per-thread indices
 
-// A-tile loader: thread tid moves 16 bytes of row tid / 8 (+ 64 p), segment tid % 8; pass p
-// moves rows 64 p + arow < BM.
-SK_HD int sk_arow(int tid) { return tid >> 3; }
-SK_HD int sk_aseg(int tid) { return tid & 7; }
-template <int BM>
-SK_HD bool sk_apass(int p, int arow) { return 64 * p + arow < BM; }
-// Element offset in Ah of the 8 halves thread (arow, aseg) loads for pass p of K-step s.
-SK_HD long sk_a_elem(const SkArgs& a, int row, int s, int aseg)
-{
-    return (long)row * a.ic + s * SK_KS + aseg * 8;
-}
-
-// B chunk of thread tid: chunk id tid = 8 * tile + c, tile = 16 ti_l + tn_l (a tile's 8 chunks
-// on 8 consecutive lanes); output column bn0 (and bn0 + 8) and input row bk0 of the K-step's
-// 64 x 256 B tile.
-SK_HD int sk_btile(int tid) { return tid >> 3; }
-SK_HD int sk_bn0(int tid) { return 16 * (sk_btile(tid) & 15) + (tid & 7); }
-SK_HD int sk_bk0(int tid) { return 16 * (sk_btile(tid) >> 4); }
-// Tile column of W_q this thread's chunk lies in for tile column block tn; a chunk beyond the
-// shard's tc tile columns is not loaded (its address is taken at column 0).
-SK_HD int sk_btn(int tid, int tn) { return 16 * tn + (sk_btile(tid) & 15); }
+// Tile column a chunk's address is taken at: a chunk past the shard's tc tile columns reads column 0.
 SK_HD int sk_bcol(int btn, int tc) { return btn < tc ? btn : 0; }
-// Tile row of the chunk in K-step s.
-SK_HD int sk_bti(int tid, int s) { return 4 * s + (sk_btile(tid) >> 4); }
 // First u32 of the chunk's K words in the trellis: tile (ti, bcol), chunk c = tid % 8.
 SK_HD long sk_b_word(int ti, int tc, int bcol, int c, int K)
 {
     return ((long)ti * tc + bcol) * (8 * K) + c * K;
-}
-
-// LDS (halves): buffer b's A tile at b * sk_buf, its B tile BM rows of SK_LD later.
-template <int BM>
-SK_HD int sk_as(int b) { return b * sk_buf<BM>(); }
-template <int BM>
-SK_HD int sk_bs(int b) { return b * sk_buf<BM>() + BM * SK_LD; }
-// A store of pass p / B stores (relative to the tile).
-SK_HD int sk_a_store(int p, int arow, int aseg) { return (64 * p + arow) * SK_LD + aseg * 8; }
-SK_HD int sk_b_store(int bn0, int bk0, int j) { return (bn0 + 8 * (j >> 1)) * SK_LD + bk0 + 8 * (j & 1); }
-// MFMA fragment reads (16 bytes = 8 halves each), relative to the tile.
-template <int BM>
-SK_HD int sk_b_frag(int wn, int nb, int lane, int h)
-{
-    return (SkCfg<BM>::NB * 16 * wn + 16 * nb + (lane & 15)) * SK_LD + 32 * h + 8 * (lane >> 4);
-}
-template <int BM>
-SK_HD int sk_a_frag(int wm, int mb, int lane, int h)
-{
-    return (SkCfg<BM>::MB * 16 * wm + 16 * mb + (lane & 15)) * SK_LD + 32 * h + 8 * (lane >> 4);
 }
 
 // ---------------------------------------------------------------- 256-row tiles: B in registers
@@ -208,8 +146,6 @@ SK_HD int sk_a_frag(int wm, int mb, int lane, int h)
 // 8 rh + 7, and its column n = l % 16 is output 16 (n / 8) + 8 ch + n % 8 of the group.  The
 // A operand of row block mb and half rh: row 16 mb + l % 16 of the wave's 128, inputs
 // 16 (l / 16) + 8 rh .. + 7 of the K-step.  Accumulator block nb = 2 g + ch.
-template <int BM>
-constexpr bool sk_rb() { return BM == 256; }
 SK_HD int sk_rb_bti(int lane, int s) { return 4 * s + (lane >> 4); }
 SK_HD int sk_rb_btn(int lane, int tn, int wn, int g) { return 16 * tn + 4 * wn + 2 * g + ((lane & 15) >> 3); }
 // A tiles: SK_RB_NBUF buffers of 256 rows x 64 halves, unpadded; a row's eight 16-byte chunks
@@ -252,10 +188,8 @@ SK_HD long sk_slot(int t, int g, int wave)
     return ((long)(t + g) * SK_WAVES + wave) * sk_acc<BM>() * 64;
 }
 
-// Epilogue LDS rows (floats): BM = 256, rows of SK_CLD per (wm, block); others, 16 rows of
-// SK_BN + 4.
+// Epilogue LDS rows (floats): rows of SK_CLD per (wm, block).
 SK_HD int sk_c256(int wm, int blk, int row, int col) { return (wm * 2 + blk) * 16 * SK_CLD + row * SK_CLD + col; }
-SK_HD int sk_cx(int row, int col) { return row * (SK_BN + 4) + col; }
 
 // ---------------------------------------------------------------- host: workspace and planning
 
@@ -277,23 +211,6 @@ inline int sk_ntn(int oc) { return (oc + SK_BN - 1) / SK_BN; }
 template <int BM>
 inline size_t sk_ws(long tiles, int G) { return sk_align((size_t)tiles * 4) + (size_t)(tiles + G) * sk_slot_bytes<BM>(); }
 
-// exl3_gemm up to this many rows runs as the one-shard grouped launch (its set-up kernel does
-// the Hadamard pass and the counter clear in one launch); above, a Hadamard pass of its own
-// that also clears the counters, then the stream-K kernel.  The workspace layout is the same.
-constexpr int SK_PREP_MAX_ROWS = 384;
-
-// Tile height of a prefill launch of `rows` rows.  Each weight is decoded once per row tile;
-// a taller tile pays that decode over more rows but MFMA work for padding rows and bigger
-// partial sums.  Measured on MI355X (17408 -> 5120, 5120 -> 17408, 5120 -> 6144): 32 is
-// fastest up to 32 rows (13-22% below 64-row tiles), 48 up to 48 (8-15% below), 64 up to
-// 64, 96 up to 96 (4-9% below 128-row tiles), 128 up to 384 (two or
-// three 128-row tiles beat one 256-row tile: more tiles, fewer stream-K partial sums per
-// tile), 256 above.
-inline int gemm_sk_bm(int rows)
-{
-    return rows <= 32 ? 32 : rows <= 48 ? 48 : rows <= 64 ? 64 : rows <= 96 ? 96 : rows <= 384 ? 128 : 256;
-}
-
 template <int BM>
 inline size_t gemm_sk_ws(int rows, int oc, int cus)
 {
@@ -301,17 +218,7 @@ inline size_t gemm_sk_ws(int rows, int oc, int cus)
 }
 
 // Counters and slots of a single-shard prefill launch.
-inline size_t sk_single_bytes(int rows, int oc, int cus)
-{
-    switch (gemm_sk_bm(rows)) {
-    case 32: return gemm_sk_ws<32>(rows, oc, cus);
-    case 48: return gemm_sk_ws<48>(rows, oc, cus);
-    case 96: return gemm_sk_ws<96>(rows, oc, cus);
-    case 64: return gemm_sk_ws<64>(rows, oc, cus);
-    case 128: return gemm_sk_ws<128>(rows, oc, cus);
-    default: return gemm_sk_ws<256>(rows, oc, cus);
-    }
-}
+inline size_t sk_single_bytes(int rows, int oc, int cus) { return gemm_sk_ws<SK_BM>(rows, oc, cus); }
 
 // Per-shard workspace of a grouped launch (several shards reading the same A): the shard's
 // activations fp16(H(A * suh)), then its share of counters and slots (each launch has at
@@ -322,26 +229,9 @@ inline size_t sk_grouped_bytes(int rows, int ic, int oc, int cus)
     return sk_align((size_t)rows * ic * 2) + sk_ws<BM>((long)((rows + BM - 1) / BM) * sk_ntn(oc), sk_gmax<BM>(cus));
 }
 
-inline size_t sk_grouped_bytes_bm(int bm, int rows, int ic, int oc, int cus)
-{
-    switch (bm) {
-    case 32: return sk_grouped_bytes<32>(rows, ic, oc, cus);
-    case 48: return sk_grouped_bytes<48>(rows, ic, oc, cus);
-    case 96: return sk_grouped_bytes<96>(rows, ic, oc, cus);
-    case 64: return sk_grouped_bytes<64>(rows, ic, oc, cus);
-    case 128: return sk_grouped_bytes<128>(rows, ic, oc, cus);
-    default: return sk_grouped_bytes<256>(rows, ic, oc, cus);
-    }
-}
-
-// The per-piece-K kernel (K = 0) exists for BM <= 128; a mixed-K group of 256-row tiles
-// is launched once per K instead.
-template <int BM>
-constexpr bool sk_has_k0() { return BM <= 128; }
-
 // One stream-K launch of the plan.
 struct SkLaunch {
-    int BM, K, cb, G;            // K = 0: each tile piece takes its shard's K
+    int K, cb, G;
     bool prep;                   // the set-up kernel (prep) runs first
     long prep_waves;
     const SkArgs* args;
@@ -373,8 +263,7 @@ inline int sk_place(SkArgs& a, int gmax, char* ws, size_t ws_bytes, const char* 
 // 32-bit words of the launch's workspace.
 inline int sk_ntiles(int rows, int oc)
 {
-    const int bm = gemm_sk_bm(rows);
-    return ((rows + bm - 1) / bm) * sk_ntn(oc);
+    return ((rows + SK_BM - 1) / SK_BM) * sk_ntn(oc);
 }
 
 // exl3_gemm's stream-K launch over one shard (Ah already transformed; its tile counters
@@ -399,31 +288,20 @@ int sk_plan_single(const uint16_t* Ah, const GemvShard& d, char* ws, size_t ws_b
     s.ntn = sk_ntn(oc);
     s.tbeg = 0;
     s.K = d.K;
-    const int bm = gemm_sk_bm(rows);
     a.ntiles = sk_ntiles(rows, oc);
     SkLaunch L = {};
-    L.BM = bm;
     L.K = d.K;
     L.cb = d.cb;
     L.args = &a;
     const char* what = "exl3_gemm (stream-K)";
-    int rc;
-    switch (bm) {
-    case 32: rc = sk_place<32>(a, sk_gmax<32>(cus), ws, ws_bytes, what, L.G); break;
-    case 48: rc = sk_place<48>(a, sk_gmax<48>(cus), ws, ws_bytes, what, L.G); break;
-    case 96: rc = sk_place<96>(a, sk_gmax<96>(cus), ws, ws_bytes, what, L.G); break;
-    case 64: rc = sk_place<64>(a, sk_gmax<64>(cus), ws, ws_bytes, what, L.G); break;
-    case 128: rc = sk_place<128>(a, sk_gmax<128>(cus), ws, ws_bytes, what, L.G); break;
-    default: rc = sk_place<256>(a, sk_gmax<256>(cus), ws, ws_bytes, what, L.G); break;
-    }
+    const int rc = sk_place<SK_BM>(a, sk_gmax<SK_BM>(cus), ws, ws_bytes, what, L.G);
     if (rc != EXL3_OK) return rc;
     return emit(static_cast<const SkLaunch&>(L));
 }
 
-// Shards that read the same A (rows x ic): per codebook (and per K where no per-piece-K
-// kernel exists), groups of up to SK_MAXSH shards; per group one set-up kernel (the
-// shards' activations, the group's tile counters) and one stream-K launch -- a single-K
-// kernel when the group's shards share K, else the per-shard-K one.
+// Shards that read the same A (rows x ic): per codebook and K, groups of up to SK_MAXSH shards;
+// per group one set-up kernel (the shards' activations, the group's tile counters) and one
+// stream-K launch.
 template <int BM, class Emit>
 int sk_plan_grouped(const uint16_t* A, const GemvShard* shards, int nshards, int rows, char* ws, size_t ws_bytes,
                     const char* what, int cus, Emit&& emit)
@@ -443,10 +321,9 @@ int sk_plan_grouped(const uint16_t* A, const GemvShard* shards, int nshards, int
         a.nks = ic / SK_KS;
         p.A = A;
         p.nblk = ic / 128;
-        int tiles = 0, K = shards[i].K;
+        int tiles = 0;
         for (int s = i; s < nshards && a.nshards < SK_MAXSH; s++) {
-            if (done[s] || shards[s].cb != shards[i].cb) continue;
-            if (!sk_has_k0<BM>() && shards[s].K != shards[i].K) continue;
+            if (done[s] || shards[s].cb != shards[i].cb || shards[s].K != shards[i].K) continue;
             const GemvShard& d = shards[s];
             if (d.K < 1 || d.K > 8) return set_error(EXL3_ERR_ARG, "%s: K=%d is not in 1..8", what, d.K);
             if (off + ah > ws_bytes)
@@ -465,7 +342,6 @@ int sk_plan_grouped(const uint16_t* A, const GemvShard* shards, int nshards, int
             e.ntn = sk_ntn(d.oc);
             e.tbeg = tiles;
             e.K = d.K;
-            if (d.K != K) K = 0;
             tiles += nrb * e.ntn;
             done[s] = true;
         }
@@ -473,8 +349,7 @@ int sk_plan_grouped(const uint16_t* A, const GemvShard* shards, int nshards, int
         p.nsh = a.nshards;
         p.counters = reinterpret_cast<uint32_t*>(ws + off);
         SkLaunch L = {};
-        L.BM = BM;
-        L.K = K;
+        L.K = shards[i].K;
         L.cb = shards[i].cb;
         L.prep = true;
         L.prep_waves = std::max<long>((long)p.nsh * rows * p.nblk, tiles);

@@ -539,76 +539,6 @@ int sk_shard_index(const SkWorld& W, const GemvShard* shards, const uint32_t* tr
     return -1;
 }
 
-// The LDS tiles of a BM-row launch: every A / B element the MFMAs read is one a store wrote,
-// and all accesses stay in their buffer's tile (independent of the piece, so checked once).
-template <int BM>
-void sk_check_lds()
-{
-    constexpr int MB = SkCfg<BM>::MB, NB = SkCfg<BM>::NB, AP = (BM + 63) / 64;
-    const int lds_halves = sk_lds<BM>() / 2;
-    for (int b = 0; b < 2; b++) {
-        std::vector<uint8_t> aw((size_t)BM * SK_KS, 0), bw((size_t)SK_BN * SK_KS, 0);
-        for (int tid = 0; tid < 64 * SK_WAVES; tid++) {
-            const int arow = sk_arow(tid), aseg = sk_aseg(tid);
-            for (int p = 0; p < AP; p++) {
-                if (!sk_apass<BM>(p, arow)) continue;
-                const int i = sk_a_store(p, arow, aseg);
-                const int row = i / SK_LD, col = i % SK_LD;
-                if (row >= BM || col + 8 > SK_KS) fail("A store outside the A tile (BM %d)", BM);
-                if (sk_as<BM>(b) + i + 8 > sk_bs<BM>(b)) fail("A store into the B tile");
-                for (int e = 0; e < 8; e++) aw[(size_t)row * SK_KS + col + e]++;
-            }
-            for (int j = 0; j < 4; j++) {
-                const int i = sk_b_store(sk_bn0(tid), sk_bk0(tid), j);
-                const int row = i / SK_LD, col = i % SK_LD;
-                if (row >= SK_BN || col + 8 > SK_KS) fail("B store outside the B tile");
-                if (sk_bs<BM>(b) + i + 8 > lds_halves) fail("B store beyond LDS");
-                for (int e = 0; e < 8; e++) bw[(size_t)row * SK_KS + col + e]++;
-            }
-        }
-        for (size_t i = 0; i < aw.size(); i++)
-            if (aw[i] != 1) fail("A tile element %zu stored %d times (BM %d)", i, aw[i], BM);
-        for (size_t i = 0; i < bw.size(); i++)
-            if (bw[i] != 1) fail("B tile element %zu stored %d times", i, bw[i]);
-        for (int wave = 0; wave < SK_WAVES; wave++) {
-            const int wm = wave / SkCfg<BM>::WN, wn = wave % SkCfg<BM>::WN;
-            for (int lane = 0; lane < 64; lane++)
-                for (int h = 0; h < 2; h++) {
-                    for (int nb = 0; nb < NB; nb++) {
-                        const int i = sk_b_frag<BM>(wn, nb, lane, h);
-                        if (i / SK_LD >= SK_BN || i % SK_LD + 8 > SK_KS) fail("B fragment outside the B tile");
-                    }
-                    for (int mb = 0; mb < MB; mb++) {
-                        const int i = sk_a_frag<BM>(wm, mb, lane, h);
-                        if (i / SK_LD >= BM || i % SK_LD + 8 > SK_KS) fail("A fragment outside the A tile (BM %d)", BM);
-                    }
-                }
-        }
-    }
-    // epilogue staging
-    const int lds_floats = sk_lds<BM>() / 4;
-    for (int wave = 0; wave < SK_WAVES; wave++) {
-        const int wm = wave / SkCfg<BM>::WN, wn = wave % SkCfg<BM>::WN;
-        for (int lane = 0; lane < 64; lane++)
-            for (int nb = 0; nb < NB; nb++)
-                for (int e = 0; e < 4; e++) {
-                    int i;
-                    if (BM == 256) i = sk_c256(wm, wn >> 1, 4 * (lane >> 4) + e, 64 * (wn & 1) + 16 * nb + (lane & 15));
-                    else i = sk_cx(4 * (lane >> 4) + e, NB * 16 * wn + 16 * nb + (lane & 15));
-                    if (i < 0 || i >= lds_floats) fail("epilogue staging store beyond LDS (BM %d)", BM);
-                }
-    }
-}
-
-// Whether a BM-row launch of K bits runs the register-B kernel (gemm_sk.hip's sk_fn and
-// sk_use_rb: 256-row tiles of one bit width, unless ORCA_EXL3_SK_RB=0).
-template <int BM>
-bool sk_replay_rb(int K)
-{
-    const char* e = getenv("ORCA_EXL3_SK_RB");
-    return sk_rb<BM>() && K > 0 && !(e && e[0] == '0');
-}
-
 // The register-B kernel's LDS: three A buffers filled by direct-to-LDS loads (each logical
 // (row, 16-byte chunk) of a K-step's 256 x 64 tile lands once, where the fragment reads look
 // for it), the two fragment-exchange buffers (each wave's stores read back by its partner
@@ -697,16 +627,14 @@ void sk_check_lds_rb()
 template <int BM>
 void sk_replay_launch(SkWorld& W, const GemvShard* shards, const SkLaunch& L, int launch)
 {
-    constexpr int MB = SkCfg<BM>::MB, NB = SkCfg<BM>::NB, AP = (BM + 63) / 64;
+    constexpr int MB = SkCfg<BM>::MB, NB = SkCfg<BM>::NB;
     const SkArgs& a = *L.args;
     const int G = L.G;
     const long units = (long)a.ntiles * a.nks;
     if (G < 1) fail("launch %d: %d workgroups", launch, G);
     if (sk_first(a, G) != units) fail("launch %d: ranges end at %ld, not %ld", launch, sk_first(a, G), units);
     if (a.q < 1) fail("launch %d: %d K-steps per workgroup", launch, a.q);
-    const bool rb = sk_replay_rb<BM>(L.K);
-    if (rb) sk_check_lds_rb();
-    else sk_check_lds<BM>();
+    sk_check_lds_rb();
     // counters and slots inside the workspace share of this launch
     ws_region(W, a.counters, (long)a.ntiles * 4, "tile counters");
     const long slot_floats = (long)(a.ntiles + G) * SK_WAVES * sk_acc<BM>() * 64;
@@ -741,18 +669,10 @@ void sk_replay_launch(SkWorld& W, const GemvShard* shards, const SkLaunch& L, in
         for (int wave = 0; wave < SK_WAVES; wave++) {
             const int wm = wave / SkCfg<BM>::WN, wn = wave % SkCfg<BM>::WN;
             for (int lane = 0; lane < 64; lane++) {
-                if (BM == 256) {
-                    const int blk = wn >> 1, half = wn & 1;
-                    for (int mb = 0; mb < MB; mb++)
-                        for (int r = 8 * half; r < 8 * half + 8; r++)
-                            store_row(m0 + 128 * wm + 16 * mb + r, 16 * tn + 8 * blk, lane);
-                } else {
-                    for (int mb = 0; mb < MB; mb++)
-                        for (int jj = 0; jj < 4; jj++) {
-                            const int j = wave + SK_WAVES * jj;
-                            store_row(m0 + 16 * mb + (j & 15), 16 * tn + 8 * (j >> 4), lane);
-                        }
-                }
+                const int blk = wn >> 1, half = wn & 1;
+                for (int mb = 0; mb < MB; mb++)
+                    for (int r = 8 * half; r < 8 * half + 8; r++)
+                        store_row(m0 + 128 * wm + 16 * mb + r, 16 * tn + 8 * blk, lane);
             }
         }
         tile_done[t]++;
@@ -773,7 +693,7 @@ void sk_replay_launch(SkWorld& W, const GemvShard* shards, const SkLaunch& L, in
             const int gi = sk_shard_index(W, shards, S.trellis);
             const int nrb = (a.rows + BM - 1) / BM;
             if (pc.tm >= nrb || pc.tn >= S.ntn || pc.t - S.tbeg >= nrb * S.ntn) fail("piece tile (%d, %d) outside shard", pc.tm, pc.tn);
-            const int KK = L.K > 0 ? L.K : S.K;
+            const int KK = L.K;
             if (KK != W.sh[gi].K) fail("piece decodes K=%d, shard has K=%d", KK, W.sh[gi].K);
             const long twords = (long)(W.sh[gi].ic / 16) * (W.sh[gi].oc / 16) * 8 * KK;
             auto load_step_rb = [&](int s) {
@@ -817,35 +737,7 @@ void sk_replay_launch(SkWorld& W, const GemvShard* shards, const SkLaunch& L, in
             };
             auto load_step = [&](int s) {
                 if (s < pc.s0 || s >= pc.s1) fail("K-step %d loaded outside the piece %d..%d", s, pc.s0, pc.s1);
-                if (rb) {
-                    load_step_rb(s);
-                    W.loads++;
-                    return;
-                }
-                for (int tid = 0; tid < 64 * SK_WAVES; tid++) {
-                    const int arow = sk_arow(tid), aseg = sk_aseg(tid);
-                    for (int p = 0; p < AP; p++) {
-                        const int row = pc.m0 + 64 * p + arow;
-                        if (sk_apass<BM>(p, arow) && row < a.rows) {
-                            const long el = sk_a_elem(a, row, s, aseg);
-                            need_in(S.Ah + el, 16, W.ah_buf[gi] >= 0 ? W.ah_buf[gi] : B_WS,
-                                    W.ah_buf[gi] >= 0 ? (long)a.rows * a.ic * 2 : (long)W.ws_bytes, "A tile load");
-                            // the 8 halves are row `row`, inside K-step s's 64 columns
-                            if (el / a.ic != row || el % a.ic < (long)s * SK_KS || el % a.ic + 8 > (long)(s + 1) * SK_KS)
-                                fail("A tile load of row %d K-step %d reads row %ld column %ld", row, s, el / a.ic, el % a.ic);
-                        }
-                    }
-                    const int btn = sk_btn(tid, pc.tn);
-                    if (btn < pc.tc) {
-                        const long wd = sk_b_word(sk_bti(tid, s), pc.tc, sk_bcol(btn, pc.tc), tid & 7, KK);
-                        need_in(S.trellis + wd, 4L * KK, B_TRELLIS + gi, twords * 4, "trellis load");
-                        // one chunk of one tile: a tile row of K-step s, a tile column of block tn
-                        const long tile = wd / (8 * KK), ti = tile / pc.tc, tj = tile % pc.tc;
-                        if (wd % (8 * KK) + KK > 8 * KK || ti < 4L * s || ti >= 4L * s + 4 || tj < 16L * pc.tn ||
-                            tj >= 16L * pc.tn + 16)
-                            fail("trellis load of K-step %d, column block %d reads tile (%ld, %ld)", s, pc.tn, ti, tj);
-                    }
-                }
+                load_step_rb(s);
                 W.loads++;
             };
             // the kernel's load order
@@ -923,16 +815,7 @@ void sk_replay_prep(SkWorld& W, const GemvShard* shards, const SkLaunch& L)
 void sk_replay_any(SkWorld& W, const GemvShard* shards, const SkLaunch& L, int launch)
 {
     if (L.prep) sk_replay_prep(W, shards, L);
-    switch (L.BM) {
-    case 32: sk_replay_launch<32>(W, shards, L, launch); break;
-    case 48: sk_replay_launch<48>(W, shards, L, launch); break;
-    case 64: sk_replay_launch<64>(W, shards, L, launch); break;
-    case 96: sk_replay_launch<96>(W, shards, L, launch); break;
-    case 128: sk_replay_launch<128>(W, shards, L, launch); break;
-    case 256: sk_replay_launch<256>(W, shards, L, launch); break;
-    default: fail("tile height %d", L.BM);
-    }
-    if (L.K == 0 && L.BM == 256) fail("per-shard-K launch of 256-row tiles");
+    sk_replay_launch<SK_BM>(W, shards, L, launch);
 }
 
 
@@ -1492,14 +1375,13 @@ int exl3r_gemm_sk(int mode, int rows, int ic, int nshards, const int* oc, const 
         std::vector<GemvShard> shards(nshards);
         long cols = 0;
         size_t ws = 0;
-        const int bm = gemm_sk_bm(rows);
         for (int i = 0; i < nshards; i++) {
             W.sh.push_back(ShardSpec{ic, oc[i], K[i], cb[i]});
             W.col0.push_back((int)cols);
             W.ah_buf.push_back(mode == 0 ? B_AH + i : -1);
             cols += oc[i];
             if (mode == 0) ws += sk_single_bytes(rows, oc[i], cus);
-            else ws += sk_grouped_bytes_bm(bm, rows, ic, oc[i], cus);
+            else ws += sk_grouped_bytes<SK_BM>(rows, ic, oc[i], cus);
         }
         W.ldc = cols;
         W.ws_bytes = ws;
@@ -1523,7 +1405,7 @@ int exl3r_gemm_sk(int mode, int rows, int ic, int nshards, const int* oc, const 
         };
         int rc;
         if (mode == 0) {
-            // above SK_PREP_MAX_ROWS exl3_gemm's Hadamard pass zeroes the launch's counters
+            // exl3_gemm's Hadamard pass zeroes the launch's counters
             // instead of a clear kernel: sk_ntiles words at the start of its workspace
             auto emit_single = [&](const SkLaunch& L) {
                 if (reinterpret_cast<const char*>(L.args->counters) != fake_ptr<char>(B_WS) ||
@@ -1535,14 +1417,8 @@ int exl3r_gemm_sk(int mode, int rows, int ic, int nshards, const int* oc, const 
             rc = sk_plan_single(fake_ptr<uint16_t>(B_AH), shards[0], fake_ptr<char>(B_WS), ws, rows, cus, emit_single);
         } else {
             const char* what = "exl3_gemm_grouped";
-            switch (bm) {
-            case 32: rc = sk_plan_grouped<32>(fake_ptr<uint16_t>(B_X), shards.data(), nshards, rows, fake_ptr<char>(B_WS), ws, what, cus, emit); break;
-            case 48: rc = sk_plan_grouped<48>(fake_ptr<uint16_t>(B_X), shards.data(), nshards, rows, fake_ptr<char>(B_WS), ws, what, cus, emit); break;
-            case 64: rc = sk_plan_grouped<64>(fake_ptr<uint16_t>(B_X), shards.data(), nshards, rows, fake_ptr<char>(B_WS), ws, what, cus, emit); break;
-            case 96: rc = sk_plan_grouped<96>(fake_ptr<uint16_t>(B_X), shards.data(), nshards, rows, fake_ptr<char>(B_WS), ws, what, cus, emit); break;
-            case 128: rc = sk_plan_grouped<128>(fake_ptr<uint16_t>(B_X), shards.data(), nshards, rows, fake_ptr<char>(B_WS), ws, what, cus, emit); break;
-            default: rc = sk_plan_grouped<256>(fake_ptr<uint16_t>(B_X), shards.data(), nshards, rows, fake_ptr<char>(B_WS), ws, what, cus, emit); break;
-            }
+            rc = sk_plan_grouped<SK_BM>(fake_ptr<uint16_t>(B_X), shards.data(), nshards, rows, fake_ptr<char>(B_WS), ws, what,
+                                        cus, emit);
         }
         if (rc != EXL3_OK) fail("plan refused: %s", exl3::g_err);
         for (int r = 0; r < rows; r++)
