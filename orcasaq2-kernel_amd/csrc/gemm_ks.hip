@@ -51,7 +51,8 @@ __global__ __launch_bounds__(512) void ks_prep_kernel(const KsPrepArgs p)
         __builtin_memcpy(&x, p.A + (long)grow * p.ic + b * 128 + 8 * l16, 16);
         __builtin_memcpy(&sg, p.suh[s] + b * 128 + 8 * l16, 16);
         float v[8], f[8];
-        had_unpack(uint4{act_pair(x.x, p.bf), act_pair(x.y, p.bf), act_pair(x.z, p.bf), act_pair(x.w, p.bf)}, v);
+        if (p.bf) x = uint4{act_pair(x.x, 1), act_pair(x.y, 1), act_pair(x.z, 1), act_pair(x.w, 1)};
+        had_unpack(x, v);
         had_unpack(sg, f);
 #pragma unroll
         for (int i = 0; i < 8; i++) v[i] *= f[i];

@@ -290,10 +290,19 @@ __global__ __launch_bounds__(G16_PREP_LANES) void gemv16_prep_kernel(const G16Pr
     const float s0 = (float)__builtin_bit_cast(_Float16, (uint16_t)(sw & 0xffffu));
     const float s1 = (float)__builtin_bit_cast(_Float16, (uint16_t)(sw >> 16));
     float v0[4], v1[4];
+    uint32_t x[4];   // loaded together: the conversion is behind a branch that would part the loads
 #pragma unroll
     for (int j = 0; j < 4; j++) {
         const int r = wv + 4 * j;
-        const uint32_t xw = r < p.rows ? act_pair(reinterpret_cast<const uint32_t*>(p.A + (long)r * p.ic + b * 128)[lane], p.bf) : 0u;
+        x[j] = r < p.rows ? reinterpret_cast<const uint32_t*>(p.A + (long)r * p.ic + b * 128)[lane] : 0u;
+    }
+    if (p.bf) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) x[j] = act_pair(x[j], 1);
+    }
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const uint32_t xw = x[j];
         v0[j] = (float)__builtin_bit_cast(_Float16, (uint16_t)(xw & 0xffffu)) * s0;
         v1[j] = (float)__builtin_bit_cast(_Float16, (uint16_t)(xw >> 16)) * s1;
     }

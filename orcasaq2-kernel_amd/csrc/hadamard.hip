@@ -33,11 +33,15 @@ __global__ __launch_bounds__(64 * HAD_WAVES) void had_r_128_kernel(
     const int lane = threadIdx.x & 15;
     const int col_blk = (int)(blk % blocks_per_row);
     float v[8];
-    const uint4 x = in[blk * 16 + lane];
-    had_unpack(uint4{act_pair(x.x, in_bf), act_pair(x.y, in_bf), act_pair(x.z, in_bf), act_pair(x.w, in_bf)}, v);
+    // loaded together: the conversion is behind a branch that would part the loads
+    uint4 x = in[blk * 16 + lane], px = {0u, 0u, 0u, 0u}, qx = px;
+    if (pre) px = pre[col_blk * 16 + lane];
+    if (post) qx = post[col_blk * 16 + lane];
+    if (in_bf) x = uint4{act_pair(x.x, 1), act_pair(x.y, 1), act_pair(x.z, 1), act_pair(x.w, 1)};
+    had_unpack(x, v);
     if (pre) {
         float p[8];
-        had_unpack(pre[col_blk * 16 + lane], p);
+        had_unpack(px, p);
 #pragma unroll
         for (int i = 0; i < 8; i++) v[i] *= p[i];
     }
@@ -47,7 +51,7 @@ __global__ __launch_bounds__(64 * HAD_WAVES) void had_r_128_kernel(
     for (int i = 0; i < 8; i++) f[i] = 0.08838834764831845f * scale;   // 1/sqrt(128)
     if (post) {
         float p[8];
-        had_unpack(post[col_blk * 16 + lane], p);
+        had_unpack(qx, p);
 #pragma unroll
         for (int i = 0; i < 8; i++) f[i] *= p[i];
     }
